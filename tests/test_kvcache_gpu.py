@@ -312,3 +312,26 @@ def test_rope_cache_writes_the_reference_layout(gpu):
     step = np.abs(got_k[~other].astype(np.int32) - want_k[~other].astype(np.int32))
     assert step.max() <= 1, f"K row off by {step.max()} f16 steps"
     assert full_scale_err(oracle.rope(q, 1, heads, hd, theta, pos), down(dq)) < 1e-5 + pos * F32EPS
+
+
+# Heads of whole float4 halves (128, 64, 80) and not (6, 2), wider than one
+# chunk of pairs (1040), and position and head counts that leave a workgroup's
+# positions, its heads in flight and the head groups ragged.
+@pytest.mark.parametrize("t,heads,hd", [(1, 1, 2), (5, 3, 6), (3, 33, 64), (9, 2, 80), (2, 3, 1040), (131, 40, 128),
+                                        (515, 9, 64)])
+@pytest.mark.parametrize("off", [0, 3, 4])
+def test_rope_of_many_rows_is_each_row_alone_and_nothing_else_moves(gpu, t, heads, hd, off):
+    first, n = 700, t * heads * hd
+    x = oracle.seq(off + n + 7, 19)
+    div = np.linspace(1.0, 8.0, hd // 2).astype(np.float32)
+    whole = up(x)
+    gpu.rope_scaled(whole, off, up(div), t, heads, hd, 10000.0, first)
+    got = down(whole)
+    want = oracle.rope(x[off:off + n], t, heads, hd, 10000.0, first, div)
+    assert full_scale_err(want, got[off:off + n]) < 1e-5 + (first + t) * F32EPS
+    assert np.array_equal(got[:off], x[:off]) and np.array_equal(got[off + n:], x[off + n:])
+    for p in {0, t // 2, t - 1}:
+        # One row, one element past a float4 boundary: the scalar form.
+        row = up(np.concatenate([[0.0], x[off + p * heads * hd: off + (p + 1) * heads * hd]]))
+        gpu.rope_scaled(row, 1, up(div), 1, heads, hd, 10000.0, first + p)
+        assert np.array_equal(down(row)[1:], got[off + p * heads * hd: off + (p + 1) * heads * hd])
