@@ -335,3 +335,27 @@ def test_rope_of_many_rows_is_each_row_alone_and_nothing_else_moves(gpu, t, head
         row = up(np.concatenate([[0.0], x[off + p * heads * hd: off + (p + 1) * heads * hd]]))
         gpu.rope_scaled(row, 1, up(div), 1, heads, hd, 10000.0, first + p)
         assert np.array_equal(down(row)[1:], got[off + p * heads * hd: off + (p + 1) * heads * hd])
+
+
+# Position tiles cut on both sides, whole and single ones; capacities whose
+# rows are whole float4s / half4s and not; a source on and off 16 bytes.
+@pytest.mark.parametrize("n,past,cap", [(1, 0, 4), (15, 3, 18), (16, 0, 16), (63, 1, 64), (64, 64, 130), (65, 62, 140),
+                                        (200, 70, 400)])
+@pytest.mark.parametrize("kv,hd", [(2, 64), (3, 128), (2, 24)])
+@pytest.mark.parametrize("src_off", [0, 1])
+def test_appended_rows_land_where_the_layouts_say(gpu, n, past, cap, kv, hd, src_off):
+    src = oracle.seq(src_off + n * kv * hd, 61)
+    rows = src[src_off:].reshape(n, kv, hd)
+    dev = up(src)
+    for f16 in (False, True):
+        for transposed in (False, True):
+            fill = oracle.seq(kv * cap * hd, 62)
+            dst = up_f16(fill) if f16 else up(fill)
+            want = down(dst).copy().reshape((kv, hd, cap) if transposed else (kv, cap, hd))
+            r = oracle.f32_to_f16(rows.ravel()).view(np.float16).reshape(n, kv, hd) if f16 else rows
+            if transposed:
+                want[:, :, past:past + n] = r.transpose(1, 2, 0)
+            else:
+                want[:, past:past + n] = r.transpose(1, 0, 2)
+            (gpu.cache_append_f16 if f16 else gpu.cache_append)(dev, src_off, dst, n, kv, hd, cap, past, transposed)
+            assert np.array_equal(down(dst), want.ravel()), (f16, transposed)

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(KB) void rope_kernel(float* x, long off, const floa
 // f32 or f16 append of n rows [n][kv*hd] into K [kv][cap][hd] or (transposed)
 // V [kv][hd][cap] at positions past..past+n-1.
 template <typename T, bool TR>
-__global__ __launch_bounds__(KB) void append_kernel(const float* src, long src_off, T* dst, int n, int kv, int hd,
+__global__ __launch_bounds__(KB) void append_kernel(const float* src, T* dst, int n, int kv, int hd,
                                                     int cap, int past) {
     const long i = (long)blockIdx.x * KB + threadIdx.x;
     const int d = kv * hd;
@@ -122,12 +122,88 @@ __global__ __launch_bounds__(KB) void append_kernel(const float* src, long src_o
     const int ti = (int)(i / d);
     const int hh = (int)((i % d) / hd);
     const int j = (int)(i % hd);
-    const float x = src[src_off + i];
+    const float x = src[i];
     const size_t at = TR ? ((size_t)hh * hd + j) * cap + past + ti : ((size_t)hh * cap + past + ti) * hd + j;
     if constexpr (sizeof(T) == 2) {
         dst[at] = __builtin_bit_cast(uint16_t, to_h(x));
     } else {
         dst[at] = x;
+    }
+}
+
+// append_kernel's K orientation eight dims a thread: two float4 in, one (f16)
+// or two (f32) 16-byte stores out, where head rows and both buffers are
+// aligned for it. 1999 rows of 8 heads of 128 into f16: 6.4 -> 4.4 us.
+template <typename T>
+__global__ __launch_bounds__(KB) void append_k8_kernel(const float* src, T* dst, unsigned total8, unsigned d8,
+                                                       unsigned hd8, int cap, int past) {
+    const unsigned i = blockIdx.x * (unsigned)KB + threadIdx.x;
+    if (i >= total8) return;
+    const unsigned ti = i / d8, c = i - ti * d8;
+    const unsigned hh = c / hd8, j = c - hh * hd8;
+    const float4* in = reinterpret_cast<const float4*>(src) + (size_t)i * 2;
+    const float4 lo = in[0], hi = in[1];
+    T* at = dst + (((size_t)hh * cap + past + ti) * hd8 + j) * 8;
+    if constexpr (sizeof(T) == 2) {
+        half8 h;
+        h[0] = to_h(lo.x), h[1] = to_h(lo.y), h[2] = to_h(lo.z), h[3] = to_h(lo.w);
+        h[4] = to_h(hi.x), h[5] = to_h(hi.y), h[6] = to_h(hi.z), h[7] = to_h(hi.w);
+        *reinterpret_cast<half8*>(at) = h;
+    } else {
+        reinterpret_cast<float4*>(at)[0] = lo;
+        reinterpret_cast<float4*>(at)[1] = hi;
+    }
+}
+
+// append_kernel's V orientation over many rows: the flat form's neighbouring
+// threads hold neighbouring dims, so each store of a wave touched 64 cache
+// rows. A workgroup takes a tile of AT_P positions by AT_D dims through LDS:
+// rows read as float4s, then four positions of one dim a thread, stored
+// together where `wide` (cap and base aligned) says so. Tiles lie on multiples
+// of AT_P positions, so a tile's stores fill whole 128-byte (f16) runs of a
+// cache row; positions outside past .. past + n - 1 are left as they are.
+// 1999 rows of 8 heads of 128 into f16: 13.6 -> 3.9 us; 173 rows: 4.6 either way (latency).
+constexpr int AT_P = 64, AT_D = 32;
+template <typename T>
+__global__ __launch_bounds__(KB) void append_vt_kernel(const float* src, T* dst, int n, int d, int cap, int past,
+                                                       int wide) {
+    __shared__ float tile[AT_D][AT_P + 1];
+    const int d0 = blockIdx.y * AT_D;
+    const int p0 = (past / AT_P + (int)blockIdx.x) * AT_P;  // the tile's first position
+#pragma unroll
+    for (int r = 0; r < AT_P * AT_D / 4 / KB; ++r) {
+        const int e = (int)threadIdx.x + r * KB;
+        const int q = e % (AT_D / 4), pl = e / (AT_D / 4);
+        const int ti = p0 + pl - past;
+        if (ti < 0 || ti >= n) continue;
+        const float4 x = *reinterpret_cast<const float4*>(src + (size_t)ti * d + d0 + 4 * q);
+        tile[4 * q][pl] = x.x;
+        tile[4 * q + 1][pl] = x.y;
+        tile[4 * q + 2][pl] = x.z;
+        tile[4 * q + 3][pl] = x.w;
+    }
+    __syncthreads();
+    typedef T quad __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int r = 0; r < AT_P * AT_D / 4 / KB; ++r) {
+        const int e = (int)threadIdx.x + r * KB;
+        const int pl = e % (AT_P / 4) * 4, dl = e / (AT_P / 4);
+        const int ti = p0 + pl - past;
+        T* at = dst + (size_t)(d0 + dl) * cap + p0 + pl;
+        quad y;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float x = tile[dl][pl + i];
+            if constexpr (sizeof(T) == 2) y[i] = __builtin_bit_cast(uint16_t, to_h(x));
+            else y[i] = x;
+        }
+        if (wide && ti >= 0 && ti + 4 <= n) {
+            *reinterpret_cast<quad*>(at) = y;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (ti + i >= 0 && ti + i < n) at[i] = y[i];
+        }
     }
 }
 
@@ -381,19 +457,35 @@ hipError_t launch_rope(float* x, long off, const float* div, int t, int heads, i
     return hipGetLastError();
 }
 
+template <typename T>
+static hipError_t launch_append_as(const float* src, T* dst, int tr, int n, int kv, int hd, int cap, int past,
+                                   hipStream_t st) {
+    const long d = (long)kv * hd, tot = n * d;
+    const bool in16 = aligned16(src) && d % 4 == 0;
+    if (!tr && in16 && hd % 8 == 0 && aligned16(dst) && tot / 8 <= 0x7fffffffL) {
+        hipLaunchKernelGGL((append_k8_kernel<T>), dim3(nblk(tot / 8)), dim3(KB), 0, st, src, dst, (unsigned)(tot / 8),
+                           (unsigned)(d / 8), (unsigned)(hd / 8), cap, past);
+        return hipGetLastError();
+    }
+    // The tiles pay from about a quarter of one in positions (below, the flat
+    // form's scattered stores are as few).
+    if (tr && in16 && d % AT_D == 0 && d / AT_D <= 65535 && n >= AT_P / 4) {
+        const int wide = cap % 4 == 0 && reinterpret_cast<uintptr_t>(dst) % (4 * sizeof(T)) == 0;
+        const dim3 g((unsigned)((past + n - 1) / AT_P - past / AT_P + 1), (unsigned)(d / AT_D));
+        hipLaunchKernelGGL((append_vt_kernel<T>), g, dim3(KB), 0, st, src, dst, n, (int)d, cap, past, wide);
+        return hipGetLastError();
+    }
+    const dim3 g(nblk(tot)), b(KB);
+    if (tr) hipLaunchKernelGGL((append_kernel<T, true>), g, b, 0, st, src, dst, n, kv, hd, cap, past);
+    else hipLaunchKernelGGL((append_kernel<T, false>), g, b, 0, st, src, dst, n, kv, hd, cap, past);
+    return hipGetLastError();
+}
+
 hipError_t launch_append(const float* src, long src_off, void* dst, int f16, int tr, int n, int kv, int hd, int cap,
                          int past, hipStream_t st) {
-    const long tot = (long)n * kv * hd;
-    if (tot == 0) return hipSuccess;
-    dim3 g(nblk(tot)), b(KB);
-    if (f16) {
-        if (tr) hipLaunchKernelGGL((append_kernel<uint16_t, true>), g, b, 0, st, src, src_off, (uint16_t*)dst, n, kv, hd, cap, past);
-        else hipLaunchKernelGGL((append_kernel<uint16_t, false>), g, b, 0, st, src, src_off, (uint16_t*)dst, n, kv, hd, cap, past);
-    } else {
-        if (tr) hipLaunchKernelGGL((append_kernel<float, true>), g, b, 0, st, src, src_off, (float*)dst, n, kv, hd, cap, past);
-        else hipLaunchKernelGGL((append_kernel<float, false>), g, b, 0, st, src, src_off, (float*)dst, n, kv, hd, cap, past);
-    }
-    return hipGetLastError();
+    if ((long)n * kv * hd == 0) return hipSuccess;
+    if (f16) return launch_append_as(src + src_off, (uint16_t*)dst, tr, n, kv, hd, cap, past, st);
+    return launch_append_as(src + src_off, (float*)dst, tr, n, kv, hd, cap, past, st);
 }
 
 hipError_t launch_rope_cache_f16(float* q, long q_off, const float* k, long k_off, const float* v, long v_off,
