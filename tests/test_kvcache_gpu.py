@@ -359,3 +359,22 @@ def test_appended_rows_land_where_the_layouts_say(gpu, n, past, cap, kv, hd, src
                 want[:, past:past + n] = r.transpose(1, 0, 2)
             (gpu.cache_append_f16 if f16 else gpu.cache_append)(dev, src_off, dst, n, kv, hd, cap, past, transposed)
             assert np.array_equal(down(dst), want.ravel()), (f16, transposed)
+
+
+# One block cut on both sides, whole blocks, several blocks; both head widths;
+# a source on 16 bytes (whole chunks) and off them (element by element).
+@pytest.mark.parametrize("n,past,cap", [(1, 5, 40), (2, 0, 32), (9, 20, 40), (32, 32, 96), (70, 3, 100), (131, 61, 192)])
+@pytest.mark.parametrize("kv,hd", [(1, 64), (3, 128)])
+@pytest.mark.parametrize("src_off", [0, 1])
+def test_rows_appended_to_a_tiled_cache_are_the_packer_s(gpu, n, past, cap, kv, hd, src_off):
+    from ttsxabe_amd.gpu import TiledCache16
+    src = {v: oracle.seq(src_off + n * kv * hd, 71 + v) for v in (0, 1)}
+    k, v = (oracle.f32_to_f16(oracle.seq(kv * cap * hd, 73 + i)) for i in (0, 1))
+    t = TiledCache16(kv, hd, cap)
+    t.data.copy_(torch.from_numpy(tiled.pack_t16(k, v, kv, hd, cap).view(np.float16)))
+    k, v = k.reshape(kv, cap, hd).copy(), v.reshape(kv, hd, cap).copy()
+    k[:, past:past + n] = oracle.f32_to_f16(src[0][src_off:]).reshape(n, kv, hd).transpose(1, 0, 2)
+    v[:, :, past:past + n] = oracle.f32_to_f16(src[1][src_off:]).reshape(n, kv, hd).transpose(1, 2, 0)
+    gpu.t16_append(up(src[0]), src_off, t, n, past, False)
+    gpu.t16_append(up(src[1]), src_off, t, n, past, True)
+    assert np.array_equal(down(t.data).view(np.uint16), tiled.pack_t16(k, v, kv, hd, cap))

@@ -381,6 +381,68 @@ __global__ __launch_bounds__(KB) void append_t16_kernel(const float* src, long s
         __builtin_bit_cast(uint16_t, to_h(src[src_off + i]));
 }
 
+// append_t16_kernel in whole fragment chunks, for sources aligned to 16 bytes
+// (the cache's blocks are). One wave takes a 32-position block's K chunk rows
+// or V dims of one kv head, each lane 16-byte stores:
+//   K: the wave's unit is (key tile T, 32 dims s), lane (key m, group g) eight
+//      dims of one key: two float4 in, one chunk out, 1 KB contiguous a wave.
+//   V: the unit is 64 dims, lane (dim quad, group g) four dims of eight keys:
+//      eight float4 in (256 contiguous bytes of four rows an instruction),
+//      four chunks out. Chunks cut by past or past + n store their own
+//      positions one by one.
+// hd / 16 units a block for K, hd / 64 for V.
+// 8192 rows of 8 heads of 128 (33 MB read, 17 written): K 26 -> 9.3 us, V
+// 31 -> 13.9 us.
+template <bool VALUE>
+__global__ __launch_bounds__(KB) void append_t16_chunks_kernel(const float* src, uint16_t* cache, int n, int kv,
+                                                               int hd, int nblk, int past, int units, int b0) {
+    const int per = VALUE ? hd / 64 : hd / 16;  // units of one block
+    const long w = (long)blockIdx.x * (KB / 64) + (threadIdx.x >> 6);
+    if (w >= units) return;
+    const int l = threadIdx.x & 63;
+    const int u = (int)w % per, hh = (int)w / per % kv, b = (int)w / per / kv + b0;
+    const int d = kv * hd;
+    uint16_t* blk = cache + ((size_t)hh * nblk + b) * 64 * hd;
+    const float* rows = src + (size_t)hh * hd;
+    if constexpr (!VALUE) {
+        const int ns = hd / 32, T = u / ns, s = u % ns;
+        const int m = l & 15, g = l >> 4;
+        const int ti = b * 32 + 8 * (m >> 2) + 4 * T + (m & 3) - past;
+        if (ti < 0 || ti >= n) return;
+        const float4* in = reinterpret_cast<const float4*>(rows + (size_t)ti * d + 32 * s + 8 * g);
+        const float4 lo = in[0], hi = in[1];
+        half8 h;
+        h[0] = to_h(lo.x), h[1] = to_h(lo.y), h[2] = to_h(lo.z), h[3] = to_h(lo.w);
+        h[4] = to_h(hi.x), h[5] = to_h(hi.y), h[6] = to_h(hi.z), h[7] = to_h(hi.w);
+        *reinterpret_cast<half8*>(blk + ((size_t)u * 64 + l) * 8) = h;
+    } else {
+        const int q = l & 15, g = l >> 4;  // dims 64u + 4q .., keys 8g ..
+        const int t0 = b * 32 + 8 * g - past;
+        float4 x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            // A position that is not appended repeats one that is.
+            const int ti = min(max(t0 + j, 0), n - 1);
+            x[j] = *reinterpret_cast<const float4*>(rows + (size_t)ti * d + 64 * u + 4 * q);
+        }
+        const int t = 4 * u + (q >> 2), c = 4 * (q & 3);
+        uint16_t* at = blk + 32 * hd + ((size_t)t * 64 + c + 16 * g) * 8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            half8 h;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) h[j] = to_h(i == 0 ? x[j].x : i == 1 ? x[j].y : i == 2 ? x[j].z : x[j].w);
+            if (t0 >= 0 && t0 + 8 <= n) {
+                *reinterpret_cast<half8*>(at + 8 * i) = h;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (t0 + j >= 0 && t0 + j < n) at[8 * i + j] = __builtin_bit_cast(uint16_t, (half_t)h[j]);
+            }
+        }
+    }
+}
+
 // The tiled twin of rope_cache_f16.
 __global__ __launch_bounds__(KB) void rope_cache_t16_kernel(float* q, long q_off, const float* k, long k_off,
                                                             const float* v, long v_off, const float* div,
@@ -529,6 +591,16 @@ hipError_t launch_append_t16(const float* src, long src_off, uint16_t* cache, in
                              int past, int value, hipStream_t st) {
     const long tot = (long)n * kv * hd;
     if (tot == 0) return hipSuccess;
+    const int b0 = past / 32;
+    const long units = (long)((past + n - 1) / 32 - b0 + 1) * kv * (value ? hd / 64 : hd / 16);
+    // Whole chunks from two rows on: a single row has one key in each chunk,
+    // and the flat form spreads it over more waves.
+    if (n > 1 && aligned16(src + src_off) && aligned16(cache) && hd % 64 == 0 && units <= 0x7fffffffL - KB) {
+        const dim3 g((unsigned)((units + KB / 64 - 1) / (KB / 64)));
+        if (value) hipLaunchKernelGGL((append_t16_chunks_kernel<true>), g, dim3(KB), 0, st, src + src_off, cache, n, kv, hd, tiled_nblk(cap), past, (int)units, b0);
+        else hipLaunchKernelGGL((append_t16_chunks_kernel<false>), g, dim3(KB), 0, st, src + src_off, cache, n, kv, hd, tiled_nblk(cap), past, (int)units, b0);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(append_t16_kernel, dim3(nblk(tot)), dim3(KB), 0, st, src, src_off, cache, n, kv, hd, cap,
                        past, value);
     return hipGetLastError();
