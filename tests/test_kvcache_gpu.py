@@ -378,3 +378,25 @@ def test_rows_appended_to_a_tiled_cache_are_the_packer_s(gpu, n, past, cap, kv, 
     gpu.t16_append(up(src[0]), src_off, t, n, past, False)
     gpu.t16_append(up(src[1]), src_off, t, n, past, True)
     assert np.array_equal(down(t.data).view(np.uint16), tiled.pack_t16(k, v, kv, hd, cap))
+
+
+@pytest.mark.parametrize("n,past,cap", [(1, 5, 40), (2, 0, 32), (9, 20, 40), (32, 32, 96), (70, 3, 100), (131, 61, 192)])
+@pytest.mark.parametrize("kv,hd", [(1, 64), (3, 128)])
+def test_rows_quantised_in_whole_chunks_are_the_rows_quantised_alone(gpu, n, past, cap, kv, hd):
+    """kv_q8_append of n rows writes the bytes that n calls of one row write
+    (element by element), at every cut of a block, with non-finite values and
+    zero blocks among them, and nothing else."""
+    from ttsxabe_amd.gpu import KvCacheQ8
+    slots, slot = 2, 1
+    k, v = (oracle.seq(n * kv * hd, 81 + i) for i in (0, 1))
+    k[:32], v[-32:] = 0.0, 0.0
+    k[40], v[7], k[-1], v[33 % v.size] = np.nan, np.inf, -np.inf, np.nan
+    whole, alone = KvCacheQ8(slots, kv, hd, cap), KvCacheQ8(slots, kv, hd, cap)
+    fill = torch.arange(whole.data.numel(), device="cuda", dtype=torch.int32).to(torch.int8)
+    whole.data.copy_(fill)
+    alone.data.copy_(fill)
+    dk, dv = up(k), up(v)
+    gpu.kv_q8_append(dk, 0, dv, 0, whole, slot, n, past)
+    for t in range(n):
+        gpu.kv_q8_append(dk, t * kv * hd, dv, t * kv * hd, alone, slot, 1, past + t)
+    assert torch.equal(whole.data, alone.data)
