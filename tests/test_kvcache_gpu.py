@@ -362,9 +362,12 @@ def test_appended_rows_land_where_the_layouts_say(gpu, n, past, cap, kv, hd, src
 
 
 # One block cut on both sides, whole blocks, several blocks; both head widths;
-# a source on 16 bytes (whole chunks) and off them (element by element).
-@pytest.mark.parametrize("n,past,cap", [(1, 5, 40), (2, 0, 32), (9, 20, 40), (32, 32, 96), (70, 3, 100), (131, 61, 192)])
-@pytest.mark.parametrize("kv,hd", [(1, 64), (3, 128)])
+# few elements (V element by element) and many (whole chunks, whose ends lie on
+# and off a chunk's eight positions); a source on 16 bytes and off them.
+@pytest.mark.parametrize("n,past,cap,kv,hd", [
+    (1, 5, 40, 1, 64), (2, 0, 32, 3, 128), (9, 20, 40, 3, 64), (32, 32, 96, 1, 128), (70, 3, 100, 3, 128),
+    (131, 61, 192, 16, 128), (256, 32, 288, 8, 128), (260, 3, 280, 16, 64), (263, 29, 300, 8, 128),
+    (41, 7, 48, 50, 128)])
 @pytest.mark.parametrize("src_off", [0, 1])
 def test_rows_appended_to_a_tiled_cache_are_the_packer_s(gpu, n, past, cap, kv, hd, src_off):
     from ttsxabe_amd.gpu import TiledCache16
@@ -380,8 +383,9 @@ def test_rows_appended_to_a_tiled_cache_are_the_packer_s(gpu, n, past, cap, kv, 
     assert np.array_equal(down(t.data).view(np.uint16), tiled.pack_t16(k, v, kv, hd, cap))
 
 
-@pytest.mark.parametrize("n,past,cap", [(1, 5, 40), (2, 0, 32), (9, 20, 40), (32, 32, 96), (70, 3, 100), (131, 61, 192)])
-@pytest.mark.parametrize("kv,hd", [(1, 64), (3, 128)])
+@pytest.mark.parametrize("n,past,cap,kv,hd", [
+    (2, 0, 32, 3, 128), (9, 20, 40, 3, 64), (70, 3, 100, 3, 128), (131, 61, 192, 8, 128), (128, 32, 160, 8, 128),
+    (130, 3, 140, 16, 64), (137, 29, 200, 8, 128), (27, 7, 48, 40, 128)])
 def test_rows_quantised_in_whole_chunks_are_the_rows_quantised_alone(gpu, n, past, cap, kv, hd):
     """kv_q8_append of n rows writes the bytes that n calls of one row write
     (element by element), at every cut of a block, with non-finite values and

@@ -48,17 +48,22 @@ __device__ __forceinline__ void rope_sc(int j, int hd, float theta, const float*
 // Kernel times, flat form -> this: 8192 rows of 32 heads of 128, 120 -> 45 us
 // (6.0 TB/s of reads and writes, what a large copy reaches); of 8 heads, 31 ->
 // 12.7; 1999 rows of 32 heads, 33 -> 11.9; 3001 rows of 8 heads, 16.0 -> 8.3.
-template <int VEC>
-__global__ __launch_bounds__(KB) void rope_kernel(float* x, long off, const float* div, int t, int heads, int hd,
-                                                  float theta, int first, int pn, int jn, int tiles, int groups,
+template <int VEC, int HD>
+__global__ __launch_bounds__(KB) void rope_kernel(float* x, long off, const float* div, int t, int heads, int hd_,
+                                                  float theta, int first, int pn_, int jn_, int tiles, int groups,
                                                   int hpb) {
     constexpr int UN = VEC == 4 ? 2 : 4;  // heads in flight
     __shared__ float2 ang[KB];
-    const int half = hd >> 1;
-    // Item = (pair chunk, head group, position tile), positions fastest.
-    const int tile = (int)(blockIdx.x % (unsigned)tiles);
-    const int grp = (int)(blockIdx.x / (unsigned)tiles % (unsigned)groups);
-    const int j0 = (int)(blockIdx.x / (unsigned)tiles / (unsigned)groups) * jn;
+    // HD > 0: the head width is known, one pair chunk, and the position tile
+    // and head group are the grid's; 0: any width, one index over all three.
+    const int hd = HD ? HD : hd_, half = hd >> 1;
+    const int jn = HD ? half : jn_, pn = HD ? KB / jn : pn_;
+    int tile = (int)blockIdx.x, grp = (int)blockIdx.y, j0 = 0;
+    if constexpr (HD == 0) {
+        tile = (int)(blockIdx.x % (unsigned)tiles);
+        grp = (int)(blockIdx.x / (unsigned)tiles % (unsigned)groups);
+        j0 = (int)(blockIdx.x / (unsigned)tiles / (unsigned)groups) * jn;
+    }
     const int jv = jn / VEC;    // vectors of one position
     const int span = pn * jv;   // threads of one head
     const int hl = (int)threadIdx.x / span, e = (int)threadIdx.x % span;
@@ -327,6 +332,23 @@ __device__ __forceinline__ uint32_t q8_code(float x, float id) {
     return (uint32_t)(uint8_t)(int8_t)(int)roundf(x * id) ^ 0x80u;
 }
 
+// The positions of past .. past + n - 1 whose eight-position V chunk is not
+// wholly appended: `lead` from past on, then `trail` up to the end. The chunk
+// kernels leave them to workgroups of their own that store element by element
+// as the flat forms do (predicated stores of a chunk's 32 values in one lane
+// held a launch of few rows up by 0.7 us).
+struct Edges {
+    int lead, trail;
+    __host__ __device__ Edges(int past, int n) {
+        const int end = past + n, up = (past + 7) / 8 * 8, down = end / 8 * 8;
+        lead = (up < end ? up : end) - past;
+        trail = down >= up ? end - down : 0;
+    }
+    __host__ __device__ int count() const { return lead + trail; }
+    // Row (of the appended ones) of edge position e.
+    __device__ int row(int e, int n) const { return e < lead ? e : n - trail + (e - lead); }
+};
+
 // append_q8_kernel in whole fragment chunks, for sources aligned to 16 bytes
 // (the cache's blocks are): the flat form stored one byte a thread and reduced
 // each block of 32 through LDS shuffles. One wave takes, of one block of one
@@ -342,11 +364,26 @@ __global__ __launch_bounds__(KB) void append_q8_chunks_kernel(const float* k, co
                                                               int n, int kv, int hd, int nblk, int past, int units,
                                                               int b0) {
     const int ns = hd / 32;  // K units of a block, and V units
+    const size_t d = (size_t)kv * hd;
+    const int uwgs = (units + KB / 64 - 1) / (KB / 64);
+    if ((int)blockIdx.x >= uwgs) {
+        const Edges ed(past, n);
+        const long i = (long)((int)blockIdx.x - uwgs) * KB + threadIdx.x;
+        const bool live = i < (long)(ed.count() * d);  // whole groups of 32 threads
+        const int ti = live ? ed.row((int)(i / (long)d), n) : 0, c = live ? (int)(i % (long)d) : 0;
+        int8_t code;
+        uint16_t db;
+        q8_block(live ? v[ti * d + c] : 0.0f, code, db);
+        if (!live) return;
+        const Q8At at = q8_at((size_t)slot * kv + c / hd, nblk, hd, past + ti, c % hd, true);
+        cache[at.code] = (char)(code ^ 0x80);
+        if ((c & 31) == 0) *reinterpret_cast<uint16_t*>(cache + at.scale) = db;
+        return;
+    }
     const int w = (int)blockIdx.x * (KB / 64) + (int)(threadIdx.x >> 6);
     if (w >= units) return;
     const int l = threadIdx.x & 63, col = l & 15, g = l >> 4;
     const int u = w % (2 * ns), hh = w / (2 * ns) % kv, b = w / (2 * ns) / kv + b0;
-    const size_t d = (size_t)kv * hd;
     char* blk = cache + (((size_t)slot * kv + hh) * nblk + b) * tq8_block_bytes(hd);
     if (u < ns) {
         const int T = u / (ns / 2), sp = u % (ns / 2);
@@ -376,7 +413,8 @@ __global__ __launch_bounds__(KB) void append_q8_chunks_kernel(const float* k, co
         float x0[8], x1[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            // A position that is not appended repeats one that is.
+            // A lane of a cut chunk repeats appended rows and stores nothing
+            // (the row maxima run over whole rows of lanes, one chunk each).
             const float* in = v + min(max(t0 + j, 0), n - 1) * d + (size_t)hh * hd + 32 * tp + col;
             x0[j] = in[0];
             x1[j] = in[16];
@@ -392,20 +430,11 @@ __global__ __launch_bounds__(KB) void append_q8_chunks_kernel(const float* k, co
         }
         char* at = blk + 32 * hd + ((size_t)tp * 64 + l) * 16;
         uint16_t* sc = reinterpret_cast<uint16_t*>(blk + 64 * hd + 2 * hd) + tp * 32 + 8 * g;
-        if (t0 >= 0 && t0 + 8 <= n) {
-            *reinterpret_cast<uint4*>(at) = make_uint4(code[0], code[1], code[2], code[3]);
-            if (col == 0) {
-                *reinterpret_cast<uint4*>(sc) = make_uint4(dh[0] | (uint32_t)dh[1] << 16, dh[2] | (uint32_t)dh[3] << 16,
-                                                           dh[4] | (uint32_t)dh[5] << 16, dh[6] | (uint32_t)dh[7] << 16);
-            }
-            return;
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            if (t0 + j < 0 || t0 + j >= n) continue;
-            at[j] = (char)(code[j >> 2] >> (8 * (j & 3)));
-            at[8 + j] = (char)(code[2 + (j >> 2)] >> (8 * (j & 3)));
-            if (col == 0) sc[j] = dh[j];
+        if (t0 < 0 || t0 + 8 > n) return;
+        *reinterpret_cast<uint4*>(at) = make_uint4(code[0], code[1], code[2], code[3]);
+        if (col == 0) {
+            *reinterpret_cast<uint4*>(sc) = make_uint4(dh[0] | (uint32_t)dh[1] << 16, dh[2] | (uint32_t)dh[3] << 16,
+                                                       dh[4] | (uint32_t)dh[5] << 16, dh[6] | (uint32_t)dh[7] << 16);
         }
     }
 }
@@ -491,8 +520,8 @@ __global__ __launch_bounds__(KB) void append_t16_kernel(const float* src, long s
 //      dims of one key: two float4 in, one chunk out, 1 KB contiguous a wave.
 //   V: the unit is 64 dims, lane (dim quad, group g) four dims of eight keys:
 //      eight float4 in (256 contiguous bytes of four rows an instruction),
-//      four chunks out. Chunks cut by past or past + n store their own
-//      positions one by one.
+//      four chunks out. Chunks cut by past or past + n are left to the
+//      workgroups past the units' (Edges).
 // hd / 16 units a block for K, hd / 64 for V.
 // 8192 rows of 8 heads of 128 (33 MB read, 17 written): K 26 -> 9.3 us, V
 // 31 -> 13.9 us.
@@ -500,11 +529,21 @@ template <bool VALUE>
 __global__ __launch_bounds__(KB) void append_t16_chunks_kernel(const float* src, uint16_t* cache, int n, int kv,
                                                                int hd, int nblk, int past, int units, int b0) {
     const int per = VALUE ? hd / 64 : hd / 16;  // units of one block
-    const long w = (long)blockIdx.x * (KB / 64) + (threadIdx.x >> 6);
+    const int d = kv * hd;
+    const int uwgs = (units + KB / 64 - 1) / (KB / 64);
+    if (VALUE && (int)blockIdx.x >= uwgs) {
+        const Edges ed(past, n);
+        const long i = (long)((int)blockIdx.x - uwgs) * KB + threadIdx.x;
+        if (i >= (long)ed.count() * d) return;
+        const int ti = ed.row((int)(i / d), n), c = (int)(i % d);
+        cache[t16_at(c / hd, nblk, hd, past + ti, c % hd, true)] =
+            __builtin_bit_cast(uint16_t, to_h(src[(size_t)ti * d + c]));
+        return;
+    }
+    const int w = (int)blockIdx.x * (KB / 64) + (int)(threadIdx.x >> 6);
     if (w >= units) return;
     const int l = threadIdx.x & 63;
-    const int u = (int)w % per, hh = (int)w / per % kv, b = (int)w / per / kv + b0;
-    const int d = kv * hd;
+    const int u = w % per, hh = w / per % kv, b = w / per / kv + b0;
     uint16_t* blk = cache + ((size_t)hh * nblk + b) * 64 * hd;
     const float* rows = src + (size_t)hh * hd;
     if constexpr (!VALUE) {
@@ -521,13 +560,12 @@ __global__ __launch_bounds__(KB) void append_t16_chunks_kernel(const float* src,
     } else {
         const int q = l & 15, g = l >> 4;  // dims 64u + 4q .., keys 8g ..
         const int t0 = b * 32 + 8 * g - past;
+        if (t0 < 0 || t0 + 8 > n) return;
         float4 x[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            // A position that is not appended repeats one that is.
-            const int ti = min(max(t0 + j, 0), n - 1);
-            x[j] = *reinterpret_cast<const float4*>(rows + (size_t)ti * d + 64 * u + 4 * q);
-        }
+        for (int j = 0; j < 8; ++j)
+            x[j] = *reinterpret_cast<const float4*>(rows + (size_t)(t0 + j) * d + 64 * u + 4 * q);
+        __builtin_amdgcn_sched_barrier(0);  // all eight rows in flight
         const int t = 4 * u + (q >> 2), c = 4 * (q & 3);
         uint16_t* at = blk + 32 * hd + ((size_t)t * 64 + c + 16 * g) * 8;
 #pragma unroll
@@ -535,13 +573,7 @@ __global__ __launch_bounds__(KB) void append_t16_chunks_kernel(const float* src,
             half8 h;
 #pragma unroll
             for (int j = 0; j < 8; ++j) h[j] = to_h(i == 0 ? x[j].x : i == 1 ? x[j].y : i == 2 ? x[j].z : x[j].w);
-            if (t0 >= 0 && t0 + 8 <= n) {
-                *reinterpret_cast<half8*>(at + 8 * i) = h;
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (t0 + j >= 0 && t0 + j < n) at[8 * i + j] = __builtin_bit_cast(uint16_t, (half_t)h[j]);
-            }
+            *reinterpret_cast<half8*>(at + 8 * i) = h;
         }
     }
 }
@@ -617,8 +649,13 @@ hipError_t launch_rope(float* x, long off, const float* div, int t, int heads, i
     const int groups = std::max(1, std::min(most, (1024 + tiles - 1) / tiles));
     const int hpb = (heads + groups * nhl - 1) / (groups * nhl) * nhl;
     const dim3 g((unsigned)((long)tiles * groups * chunks)), b(KB);
-    if (vec == 4) hipLaunchKernelGGL((rope_kernel<4>), g, b, 0, st, x, off, div, t, heads, hd, theta, first, pn, jn, tiles, groups, hpb);
-    else hipLaunchKernelGGL((rope_kernel<1>), g, b, 0, st, x, off, div, t, heads, hd, theta, first, pn, jn, tiles, groups, hpb);
+#define ROPE(V, H, G) \
+    hipLaunchKernelGGL((rope_kernel<V, H>), G, b, 0, st, x, off, div, t, heads, hd, theta, first, pn, jn, tiles, groups, hpb)
+    if (vec == 4 && hd == 128) ROPE(4, 128, dim3(tiles, groups));
+    else if (vec == 4 && hd == 64) ROPE(4, 64, dim3(tiles, groups));
+    else if (vec == 4) ROPE(4, 0, g);
+    else ROPE(1, 0, g);
+#undef ROPE
     return hipGetLastError();
 }
 
@@ -677,9 +714,10 @@ hipError_t launch_append_q8(const float* k, long k_off, const float* v, long v_o
     if (tot == 0) return hipSuccess;
     const int b0 = past / 32;
     const long units = (long)((past + n - 1) / 32 - b0 + 1) * kv * (hd / 16);
-    // As launch_append_t16: whole chunks from two rows on.
-    if (n > 1 && aligned16(k + k_off) && aligned16(cache) && hd % 64 == 0 && units <= 0x7fffffffL - KB) {
-        const dim3 g((unsigned)((units + KB / 64 - 1) / (KB / 64)));
+    // As launch_append_t16, from half as many elements (there are two areas):
+    // 60 rows of 8 x 128, 3.59 us in chunks and 3.44 flat; 173 rows, 3.64 and 3.87.
+    if (tot >= 1L << 17 && aligned16(k + k_off) && aligned16(cache) && hd % 64 == 0 && units <= 0x7fffffffL - KB) {
+        const dim3 g((unsigned)((units + KB / 64 - 1) / (KB / 64)) + nblk((long)Edges(past, n).count() * kv * hd));
         hipLaunchKernelGGL(append_q8_chunks_kernel, g, dim3(KB), 0, st, k + k_off, v + v_off, cache, slot, n, kv, hd, tiled_nblk(cap), past, (int)units, b0);
         return hipGetLastError();
     }
@@ -704,10 +742,12 @@ hipError_t launch_append_t16(const float* src, long src_off, uint16_t* cache, in
     if (tot == 0) return hipSuccess;
     const int b0 = past / 32;
     const long units = (long)((past + n - 1) / 32 - b0 + 1) * kv * (value ? hd / 64 : hd / 16);
-    // Whole chunks from two rows on: a single row has one key in each chunk,
-    // and the flat form spreads it over more waves.
-    if (n > 1 && aligned16(src + src_off) && aligned16(cache) && hd % 64 == 0 && units <= 0x7fffffffL - KB) {
-        const dim3 g((unsigned)((units + KB / 64 - 1) / (KB / 64)));
+    // Whole chunks once the flat form would take about 1024 workgroups (V) or
+    // from two rows on (K, whose chunks are one key's): 173 rows of 8 x 128, V
+    // 2.66 us in chunks and 2.57 flat; 300 rows, 3.17 and 3.31; K even at 29.
+    if ((value ? tot >= 1L << 18 : n > 1) && aligned16(src + src_off) && aligned16(cache) && hd % 64 == 0 && units <= 0x7fffffffL - KB) {
+        const dim3 g((unsigned)((units + KB / 64 - 1) / (KB / 64)) +
+                     (value ? nblk((long)Edges(past, n).count() * kv * hd) : 0u));
         if (value) hipLaunchKernelGGL((append_t16_chunks_kernel<true>), g, dim3(KB), 0, st, src + src_off, cache, n, kv, hd, tiled_nblk(cap), past, (int)units, b0);
         else hipLaunchKernelGGL((append_t16_chunks_kernel<false>), g, dim3(KB), 0, st, src + src_off, cache, n, kv, hd, tiled_nblk(cap), past, (int)units, b0);
         return hipGetLastError();
