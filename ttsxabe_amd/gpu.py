@@ -111,8 +111,9 @@ def _check(status: int):
 
 
 def _p(t):
-    """Device pointer of a tensor (None -> NULL)."""
-    return None if t is None else C.c_void_p(t.data_ptr())
+    """Device pointer of a tensor (None -> NULL), as the plain integer the
+    declared argument types take."""
+    return None if t is None else t.data_ptr()
 
 
 def _n(t):
@@ -120,14 +121,13 @@ def _n(t):
 
 
 def _need(t, dtypes, what):
-    if t is None:
+    if t is None or (t.is_cuda and t.dtype in dtypes and t.is_contiguous()):
         return
     if not t.is_cuda:
         raise InvalidArgument(f"{what} is not a device tensor")
     if t.dtype not in dtypes:
         raise InvalidArgument(f"{what} has dtype {t.dtype}, wanted one of {dtypes}")
-    if not t.is_contiguous():
-        raise InvalidArgument(f"{what} is not contiguous")
+    raise InvalidArgument(f"{what} is not contiguous")
 
 
 _F32 = (torch.float32,)
@@ -227,7 +227,10 @@ class Gpu:
         self._L = L
 
     def _stream(self):
-        return C.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
+        # The current stream's handle without a Stream object: a call of a few
+        # launches is as long as its host work (three calls of the f32 prompt
+        # layer took 25.2 us of host work with the ctypes and Stream objects, 17.2 us without).
+        return torch._C._cuda_getCurrentRawStream(self.device.index)
 
     # ------------------------------------------------------------- prefill
 
@@ -240,7 +243,7 @@ class Gpu:
         _need(v, kdt, "v")
         out = torch.empty(max(tq * heads * head_dim, 1), dtype=torch.float32, device=self.device)
         _check(fn(self._stream(), _p(q), _n(q), _p(k), _n(k), _p(v), _n(v), _p(out), tq * heads * head_dim, tq, past,
-                  heads, kv_heads, head_dim, cap, C.c_float(scale), int(bool(causal))))
+                  heads, kv_heads, head_dim, cap, scale, int(bool(causal))))
         return out[: tq * heads * head_dim]
 
     def flash_attn(self, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale, causal):
@@ -259,7 +262,7 @@ class Gpu:
         n = t * heads * head_dim
         out = torch.empty(max(n, 1), dtype=torch.float16, device=self.device)
         _check(self._L.llmtie_flash_attn_rows(self._stream(), _p(qkv), _n(qkv), _p(out), n, t, heads, head_dim,
-                                              C.c_float(scale)))
+                                              scale))
         return out[:n]
 
     # -------------------------------------------------------------- decode
@@ -272,7 +275,7 @@ class Gpu:
         n = heads * head_dim
         out = torch.empty(n, dtype=torch.float32, device=self.device)
         _check(self._L.llmtie_attn_decode_f16(self._stream(), _p(q), _n(q), _p(k), _n(k), _p(v), _n(v), heads,
-                                              kv_heads, head_dim, tk, cap, C.c_float(scale), int(bool(scale_q)),
+                                              kv_heads, head_dim, tk, cap, scale, int(bool(scale_q)),
                                               scratch.handle, _p(out), n))
         return out
 
@@ -288,7 +291,7 @@ class Gpu:
         if out is None:
             out = torch.empty(n, dtype=torch.float32, device=self.device)
         _check(self._L.llmtie_attn_decode_f16_noalloc(self._stream(), _p(q), _n(q), _p(k), _n(k), _p(v), _n(v),
-                                                      heads, kv_heads, head_dim, tk, cap, C.c_float(scale),
+                                                      heads, kv_heads, head_dim, tk, cap, scale,
                                                       int(bool(scale_q)), _p(out), _n(out)))
         return out
 
@@ -307,7 +310,7 @@ class Gpu:
         out = torch.empty(n, dtype=torch.float32, device=self.device)
         twin = Q8(torch.empty(n + (n // 32) * 4, dtype=torch.int8, device=self.device), 1, n)
         _check(self._L.llmtie_attn_decode_f16_q(self._stream(), _p(q), _n(q), _p(k), _n(k), _p(v), _n(v), heads,
-                                                kv_heads, head_dim, tk, cap, C.c_float(scale), int(bool(scale_q)),
+                                                kv_heads, head_dim, tk, cap, scale, int(bool(scale_q)),
                                                 scratch.handle, _p(out), n, _p(twin.buf), twin.buf.numel()))
         return out, twin
 
@@ -319,7 +322,7 @@ class Gpu:
         _need(v, _H16, "v")
         _need(out, _F32, "out")
         _check(self._L.llmtie_attn_decode_f16_q_row(self._stream(), _p(q), _n(q), q_off, _p(k), _n(k), _p(v), _n(v),
-                                                    heads, kv_heads, head_dim, tk, cap, C.c_float(scale),
+                                                    heads, kv_heads, head_dim, tk, cap, scale,
                                                     int(bool(scale_q)), scratch.handle, _p(out), _n(out),
                                                     _p(twin.buf), twin.rows, twin.k, row))
 
@@ -331,7 +334,7 @@ class Gpu:
         n = heads * head_dim
         out = torch.empty(n, dtype=torch.float32, device=self.device)
         _check(self._L.llmtie_attn_decode(self._stream(), _p(q), _n(q), _p(k), _n(k), _p(v), _n(v), heads, kv_heads,
-                                          head_dim, tk, cap, C.c_float(scale), int(bool(scale_q)), scratch.handle,
+                                          head_dim, tk, cap, scale, int(bool(scale_q)), scratch.handle,
                                           _p(out), n))
         return out
 
@@ -347,7 +350,7 @@ class Gpu:
             out = torch.empty(max(nseq * n, 1), dtype=torch.float32, device=self.device)
         _check(self._L.llmtie_attn_decode_q8_batch(
             self._stream(), _p(q), _n(q), _p(cache.data), _n(cache.data), cache.slots, _p(tk_dev), _p(slot_dev),
-            nseq, max_tk, heads, cache.kv_heads, cache.head_dim, cache.cap, C.c_float(scale), int(bool(scale_q)),
+            nseq, max_tk, heads, cache.kv_heads, cache.head_dim, cache.cap, scale, int(bool(scale_q)),
             scratch.handle, _p(out), _n(out)))
         return out[: nseq * n]
 
@@ -360,7 +363,7 @@ class Gpu:
         if out is None:
             out = torch.empty(n, dtype=torch.float32, device=self.device)
         _check(self._L.llmtie_attn_decode_t16(self._stream(), _p(q), _n(q), _p(cache.data), _n(cache.data), heads,
-                                              cache.kv_heads, cache.head_dim, tk, cache.cap, C.c_float(scale),
+                                              cache.kv_heads, cache.head_dim, tk, cache.cap, scale,
                                               int(bool(scale_q)), scratch.handle, _p(out), _n(out)))
         return out
 
@@ -371,7 +374,7 @@ class Gpu:
         _need(out, _F32, "out")
         _check(self._L.llmtie_attn_decode_t16_q_row(
             self._stream(), _p(q), _n(q), q_off, _p(cache.data), _n(cache.data), heads, cache.kv_heads,
-            cache.head_dim, tk, cache.cap, C.c_float(scale), int(bool(scale_q)), scratch.handle, _p(out), _n(out),
+            cache.head_dim, tk, cache.cap, scale, int(bool(scale_q)), scratch.handle, _p(out), _n(out),
             None if twin is None else _p(twin.buf), 0 if twin is None else twin.rows,
             0 if twin is None else twin.k, row))
 
@@ -382,7 +385,7 @@ class Gpu:
         out = torch.empty(max(n, 1), dtype=torch.float32, device=self.device)
         _check(self._L.llmtie_flash_attn_t16(self._stream(), _p(q), _n(q), _p(cache.data), _n(cache.data), _p(out),
                                              n, tq, past, heads, cache.kv_heads, cache.head_dim, cache.cap,
-                                             C.c_float(scale), int(bool(causal))))
+                                             scale, int(bool(causal))))
         return out[:n]
 
     def t16_append(self, src, src_off, cache: TiledCache16, n, past, value):
@@ -397,7 +400,7 @@ class Gpu:
             _need(t, _F32, w)
         _check(self._L.llmtie_t16_rope_cache(self._stream(), _p(q), _n(q), q_off, _p(k), _n(k), k_off, _p(v), _n(v),
                                              v_off, _p(freq_div), heads, cache.kv_heads, cache.head_dim,
-                                             C.c_float(theta), pos, _p(cache.data), _n(cache.data), cache.cap))
+                                             theta, pos, _p(cache.data), _n(cache.data), cache.cap))
 
     def t16_grow(self, src: TiledCache16, dst: TiledCache16, live):
         """cache_grow_f16 (device.rs:3152) between tiled caches."""
@@ -422,7 +425,7 @@ class Gpu:
         _need(x, _F32, "x")
         _need(freq_div, _F32, "freq_div")
         _check(self._L.llmtie_rope(self._stream(), _p(x), _n(x), off, _p(freq_div), t, heads, head_dim,
-                                   C.c_float(theta), first))
+                                   theta, first))
 
     def cache_append(self, src, src_off, dst, n, kv_heads, head_dim, cap, past, transposed):
         """device.rs:3013."""
@@ -447,7 +450,7 @@ class Gpu:
         _need(kc, _H16, "kc")
         _need(vc, _H16, "vc")
         _check(self._L.llmtie_rope_cache_f16(self._stream(), _p(q), _n(q), q_off, _p(k), _n(k), k_off, _p(v), _n(v),
-                                             v_off, _p(freq_div), heads, kv_heads, head_dim, C.c_float(theta), pos,
+                                             v_off, _p(freq_div), heads, kv_heads, head_dim, theta, pos,
                                              _p(kc), _p(vc), min(_n(kc), _n(vc)), cap))
 
     def cache_grow(self, src, dst, kv_heads, head_dim, cap, new_cap, live, transposed):
@@ -478,5 +481,5 @@ class Gpu:
             _need(t, _F32, w)
         _check(self._L.llmtie_rope_cache_q8(self._stream(), _p(q), _n(q), q_off, _p(k), _n(k), k_off, _p(v), _n(v),
                                             v_off, _p(freq_div), heads, cache.kv_heads, cache.head_dim,
-                                            C.c_float(theta), pos, _p(cache.data), _n(cache.data), cache.slots, slot,
+                                            theta, pos, _p(cache.data), _n(cache.data), cache.slots, slot,
                                             cache.cap))
