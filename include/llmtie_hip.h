@@ -129,6 +129,24 @@ int llmtie_flash_attn_f16(void* stream, const float* q, size_t q_len, const uint
                           const uint16_t* v, size_t v_len, float* out, size_t out_len, size_t tq, size_t past,
                           size_t heads, size_t kv_heads, size_t head_dim, size_t cap, float scale, int causal);
 
+/* No counterpart in the reference: the f16 prefills with a workspace, for
+ * launches of few rows over many keys (a turn of a long conversation), whose
+ * keys are then cut into runs attended by workgroups of their own and merged
+ * in a second launch. llmtie_flash_attn_workspace gives the floats such a call
+ * needs (0: the shape is not split, and no workspace is needed). The workspace
+ * is written and read on `stream` by this call alone and may be reused or
+ * freed in stream order after it; concurrent calls need one each. `ws` NULL is
+ * the plain call. A workspace shorter than needed is refused as
+ * LLMTIE_SLICE_OVERRUN. It is 16-byte aligned. */
+size_t llmtie_flash_attn_workspace(size_t tq, size_t past, size_t heads, size_t kv_heads, size_t head_dim);
+int llmtie_flash_attn_f16_ws(void* stream, const float* q, size_t q_len, const uint16_t* k, size_t k_len,
+                             const uint16_t* v, size_t v_len, float* out, size_t out_len, size_t tq, size_t past,
+                             size_t heads, size_t kv_heads, size_t head_dim, size_t cap, float scale, int causal,
+                             float* ws, size_t ws_len);
+int llmtie_flash_attn_t16_ws(void* stream, const float* q, size_t q_len, const uint16_t* cache, size_t cache_len,
+                             float* out, size_t out_len, size_t tq, size_t past, size_t heads, size_t kv_heads,
+                             size_t head_dim, size_t cap, float scale, int causal, float* ws, size_t ws_len);
+
 /* Gpu::flash_attn_rows (device.rs:5812): non-causal attention over a stacked
  * [t, 3*heads*head_dim] q/k/v product, scale on q, context as f16 bits
  * [t, heads*head_dim]. head_dim 64. The rows are read where they lie and

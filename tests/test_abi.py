@@ -189,3 +189,21 @@ def test_the_decode_boundary_accepts_its_documented_superset():
 def test_a_scratch_with_no_lost_head_reports_ok():
     L = _lib.lib()
     assert L.llmtie_decode_scratch_status(NULL) == 0
+
+
+def test_the_prefill_workspace_is_asked_for_where_keys_outnumber_rows():
+    L = _lib.lib()
+    need = L.llmtie_flash_attn_workspace
+    # A turn of a long conversation splits; whole runs of (hd + 2) floats a (row, head).
+    n = need(173, 3011, 32, 8, 128)
+    assert n and n % (173 * 32 * 130) == 0 and n // (173 * 32 * 130) <= 32
+    # First prompts, short contexts and launches that fill the chip do not.
+    for shape in [(512, 0, 32, 8, 128), (2048, 0, 32, 8, 128), (8192, 0, 32, 8, 128), (64, 448, 32, 8, 128),
+                  (2000, 6000, 32, 8, 128), (0, 4000, 32, 8, 128)]:
+        assert need(*shape) == 0, shape
+    # Nor do shapes the prefill refuses, up to the top of size_t.
+    for shape in [(16, 3000, 32, 8, 96), (16, 3000, 33, 8, 128), (16, 3000, 32, 0, 128), (16, W - 8, 32, 8, 128),
+                  (W - 1, 3000, 32, 8, 128), (16, 3000, 2**60, 2**60, 128)]:
+        assert need(*shape) == 0, shape
+    # Never more than about 800 workgroups' 64 rows of partials.
+    assert max(need(t, p, 32, 8, 128) for t in range(1, 700, 13) for p in range(0, 8000, 533)) <= 800 * 64 * 130

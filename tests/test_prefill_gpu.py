@@ -268,3 +268,56 @@ def test_the_long_prefill_at_its_full_shape(gpu, monkeypatch):
         err = np.abs(want - got[r * n:(r + 1) * n])
         worst = float((err / tol).max())
         assert worst < 0.5, f"row {r}: worst error {worst} of its tolerance"
+
+
+# Few rows over many keys, cut into runs (the workspace says so): query groups
+# of 1, 2, 4 and 8, both head widths, rows that leave a position block ragged,
+# a last tile cut anywhere, causal and full; runs that some rows see nothing of
+# (causal rows from position 0).
+@pytest.mark.parametrize("heads,kv,hd,causal,tq,past,cap", [
+    (8, 2, 128, True, 20, 1501, 1536), (4, 4, 64, True, 70, 1000, 1070), (6, 3, 128, False, 1, 2047, 2048),
+    (16, 2, 64, False, 17, 911, 930), (8, 2, 128, True, 16, 3008, 3024), (4, 1, 128, True, 1500, 0, 1504)])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_a_split_prefill_is_the_whole_one(gpu, heads, kv, hd, causal, tq, past, cap, tiled):
+    from ttsxabe_amd.gpu import TiledCache16
+    assert gpu._flash_ws(tq, past, heads, kv, hd) is not None, "the shape is meant to split"
+    tk, n = past + tq, heads * hd
+    scale = float(np.float32(hd) ** np.float32(-0.5))
+    q = oracle.seq(tq * n, 181) * np.float32(4.0)
+    k, v = (oracle.through_f16(oracle.seq(kv * tk * hd, s)) for s in (182, 183))
+    kc, vc = caches(k, v, kv, tk, cap, hd)
+    k16, v16 = up_f16(kc), up_f16(vc)
+    # What lies past the keys never reaches the context.
+    k16.view(kv, cap, hd)[:, tk:] = float("nan")
+    v16.view(kv, hd, cap)[:, :, tk:] = float("nan")
+    dq = up(q)
+    L = gpu._L
+    if tiled:
+        t = TiledCache16(kv, hd, cap, zero=False)
+        t.data.fill_(float("nan"))
+        gpu.t16_from_ref(k16, v16, t, tk)
+        got = down(gpu.flash_attn_t16(dq, t, tq, past, heads, scale, causal))
+        again = down(gpu.flash_attn_t16(dq, t, tq, past, heads, scale, causal))
+    else:
+        got = down(gpu.flash_attn_f16(dq, k16, v16, tq, past, heads, kv, hd, cap, scale, causal))
+        again = down(gpu.flash_attn_f16(dq, k16, v16, tq, past, heads, kv, hd, cap, scale, causal))
+    assert np.array_equal(got, again)
+    whole = down(gpu._flash(L.llmtie_flash_attn_f16, dq, k16, v16, tq, past, heads, kv, hd, cap, scale, causal,
+                            (torch.float16,)))
+    # Both round each probability to f16 once, against different references:
+    # at most 2^-11 of it each way, so of the largest value in the context.
+    assert np.abs(got - whole).max() <= 2.0 ** -10 * np.abs(v).max()
+    want, spread = oracle.prefill_ref(q, n, kc, vc, tq, past, heads, kv, hd, cap, scale, causal)
+    tol = 2e-4 + 1e-2 * np.abs(want) + 1e-2 * spread
+    assert float((np.abs(want - got) / tol).max()) < 0.5
+
+
+def test_a_workspace_too_short_for_its_split_is_refused(gpu):
+    from ttsxabe_amd.gpu import SliceOverrun, _n, _p
+    heads, kv, hd, tq, past, cap = 8, 2, 128, 20, 1500, 1536
+    q = torch.zeros(tq * heads * hd, device="cuda")
+    c = torch.zeros(kv * cap * hd, dtype=torch.float16, device="cuda")
+    ws = gpu._flash_ws(tq, past, heads, kv, hd)[:-1]
+    with pytest.raises(SliceOverrun):
+        gpu._flash(gpu._L.llmtie_flash_attn_f16_ws, q, c, c, tq, past, heads, kv, hd, cap, 1.0, True,
+                   (torch.float16,), _p(ws), _n(ws))

@@ -35,6 +35,9 @@ SIGNATURES = {
     "llmtie_supports_flash": (I, [SZ, SZ, SZ]),
     "llmtie_flash_attn": (I, [P, P, SZ, P, SZ, P, SZ, P, SZ, SZ, SZ, SZ, SZ, SZ, SZ, F, I]),
     "llmtie_flash_attn_f16": (I, [P, P, SZ, P, SZ, P, SZ, P, SZ, SZ, SZ, SZ, SZ, SZ, SZ, F, I]),
+    "llmtie_flash_attn_workspace": (SZ, [SZ, SZ, SZ, SZ, SZ]),
+    "llmtie_flash_attn_f16_ws": (I, [P, P, SZ, P, SZ, P, SZ, P, SZ, SZ, SZ, SZ, SZ, SZ, SZ, F, I, P, SZ]),
+    "llmtie_flash_attn_t16_ws": (I, [P, P, SZ, P, SZ, P, SZ, SZ, SZ, SZ, SZ, SZ, SZ, F, I, P, SZ]),
     "llmtie_flash_attn_rows": (I, [P, P, SZ, P, SZ, SZ, SZ, SZ, F]),
     "llmtie_attn_decode_f16": (I, [P, P, SZ, P, SZ, P, SZ, SZ, SZ, SZ, SZ, SZ, F, I, P, P, SZ]),
     "llmtie_attn_decode_f16_noalloc": (I, [P, P, SZ, P, SZ, P, SZ, SZ, SZ, SZ, SZ, SZ, F, I, P, SZ]),

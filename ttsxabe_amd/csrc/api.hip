@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -171,9 +172,48 @@ int pick_nqt(size_t tq, size_t heads, int gb, bool staged = false) {
     return 1;
 }
 
+// Runs the tiles of each position block of a prefill off an f16 cache are cut
+// into (1: not split), one workgroup each: the cheapest under a model of the
+// launch fitted to MI355X, in microseconds at head_dim 128. A workgroup's 64-key
+// tile takes 0.95 alone on its compute unit and 1.5 beside a second one (two
+// fit); a third waits. Splitting adds the merge's launch and the partials'
+// traffic, so few rows over many keys split far and many rows or few keys not
+// at all. Measured, split / not: 173 rows after 3011 positions of 32/8/128, 28 /
+// 47 us; 16 after 3000, 14.6 / 44; 100 after 7000, 28 / 95; 40 after 1000,
+// 13.1 / 19.5. Where the model keeps one run, two or three measured slower: 300
+// rows after 700, 24 / 20; 64 after 448, 11.6 / 11.1; 400 after 1500 of
+// 40/40/128, 49 / 42; 2000 first rows of 8/2/128, 33-35 / 34.
+constexpr size_t PREFILL_MAX_SPLITS = 32;
+size_t plan_prefill_splits(size_t tq, size_t past, size_t heads, size_t kv_heads, size_t hd) {
+    if (getenv("LLMTIE_PREFILL_NQT")) return 1;
+    const size_t group = heads / kv_heads;
+    const size_t gb = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
+    const size_t pb = 16 * (4 / gb);
+    const double cus = compute_units();
+    const double items = (double)((tq + pb - 1) / pb) * (double)(heads / gb);
+    if (items > 2 * cus) return 1;
+    const size_t tiles = (past + tq + 63) / 64;
+    if (tiles <= 8) return 1;  // no shape measured gains; the Python binding does not ask either
+    const double tile_us = hd == 128 ? 1.0 : 0.7;
+    // One run's partials written and read, and its share of the merge's chain.
+    const double run_us = (double)(tq * heads * hd) * 8.0 / 5e6 + 0.1;
+    size_t best = 1;
+    double least = 0.0;
+    for (size_t n = 1; n <= PREFILL_MAX_SPLITS && n <= tiles; ++n) {
+        const double load = items * (double)n / cus;
+        const double period = load <= 1.0 ? 0.95 : load <= 2.0 ? 0.95 + 0.55 * (load - 1.0) : 0.75 * std::ceil(load);
+        const double us = (double)((tiles + n - 1) / n) * period * tile_us + (n > 1 ? 4.5 + (double)n * run_us : 0.0);
+        if (n == 1 || us < least) {
+            best = n;
+            least = us;
+        }
+    }
+    return best;
+}
+
 int prefill_common(void* stream, int kind, const float* q, size_t q_len, const void* k, size_t k_len, const void* v,
                    size_t v_len, float* out, size_t out_len, size_t tq, size_t past, size_t heads, size_t kv_heads,
-                   size_t hd, size_t cap, float scale, int causal) {
+                   size_t hd, size_t cap, float scale, int causal, float* ws = nullptr, size_t ws_len = 0) {
     if (!(hd == 64 || hd == 128) || kv_heads == 0 || heads % kv_heads != 0) return unsupported(hd, heads, kv_heads);
     if (sadd(past, tq) > cap) return overrun_cache(sadd(past, tq), cap);
     if (int r = over_int(smul(heads, hd), cap)) return r;
@@ -206,7 +246,15 @@ int prefill_common(void* stream, int kind, const float* q, size_t q_len, const v
     a.os = (int)(heads * hd);
     a.scale_q = 0;
     a.v_bytes = v_len * (kind == PF_F32 ? 4 : 2);
-    const int nqt = pick_nqt(tq, heads, gb, kind == PF_F32);
+    int nqt = pick_nqt(tq, heads, gb, kind == PF_F32);
+    const size_t splits = ws ? plan_prefill_splits(tq, past, heads, kv_heads, hd) : 1;
+    if (splits > 1) {
+        const size_t need = smul(smul(splits, tq, heads), hd + 2);
+        if (ws_len < need) return overrun_slice(need, ws_len);
+        a.splits = (int)splits;
+        a.ws = ws;
+        nqt = 1;
+    }
     return launched("flash_attn", launch_prefill((int)hd, kind, nqt, a, S(stream)));
 }
 
@@ -493,6 +541,25 @@ int llmtie_flash_attn_f16(void* stream, const float* q, size_t q_len, const uint
     if (cap % 2 != 0) return odd_cap(cap);
     return prefill_common(stream, PF_F16, q, q_len, k, k_len, v, v_len, out, out_len, tq, past, heads, kv_heads,
                           head_dim, cap, scale, causal);
+}
+
+size_t llmtie_flash_attn_workspace(size_t tq, size_t past, size_t heads, size_t kv_heads, size_t head_dim) {
+    // Shapes the prefill itself refuses need none.
+    if (!llmtie_supports_flash(head_dim, heads, kv_heads) || tq == 0 || sadd(past, tq) > IMAX ||
+        smul(heads, head_dim) > IMAX || smul(tq, heads, head_dim) > (size_t)1 << 40)
+        return 0;
+    const size_t n = plan_prefill_splits(tq, past, heads, kv_heads, head_dim);
+    return n > 1 ? smul(smul(n, tq, heads), head_dim + 2) : 0;
+}
+
+int llmtie_flash_attn_f16_ws(void* stream, const float* q, size_t q_len, const uint16_t* k, size_t k_len,
+                             const uint16_t* v, size_t v_len, float* out, size_t out_len, size_t tq, size_t past,
+                             size_t heads, size_t kv_heads, size_t head_dim, size_t cap, float scale, int causal,
+                             float* ws, size_t ws_len) {
+    if (!(head_dim == 64 || head_dim == 128)) return unsupported(head_dim, heads, kv_heads);
+    if (cap % 2 != 0) return odd_cap(cap);
+    return prefill_common(stream, PF_F16, q, q_len, k, k_len, v, v_len, out, out_len, tq, past, heads, kv_heads,
+                          head_dim, cap, scale, causal, ws, ws_len);
 }
 
 int llmtie_flash_attn_rows(void* stream, const float* qkv, size_t qkv_len, uint16_t* out, size_t out_len, size_t t,
@@ -928,16 +995,23 @@ int llmtie_attn_decode_t16_q_row(void* stream, const float* q, size_t q_len, siz
                          twin_k, twin != nullptr);
 }
 
-int llmtie_flash_attn_t16(void* stream, const float* q, size_t q_len, const uint16_t* cache, size_t cache_len,
-                          float* out, size_t out_len, size_t tq, size_t past, size_t heads, size_t kv_heads,
-                          size_t head_dim, size_t cap, float scale, int causal) {
+int llmtie_flash_attn_t16_ws(void* stream, const float* q, size_t q_len, const uint16_t* cache, size_t cache_len,
+                             float* out, size_t out_len, size_t tq, size_t past, size_t heads, size_t kv_heads,
+                             size_t head_dim, size_t cap, float scale, int causal, float* ws, size_t ws_len) {
     int r = t16_checks(head_dim, heads, kv_heads, cap, cache_len);
     if (r != LLMTIE_OK) return r;
     // The tiled cache holds both areas in one buffer; the length checks of the
     // shared path are satisfied by passing the whole-cache extent for both.
     const size_t ext = smul(kv_heads, cap, head_dim);
     return prefill_common(stream, PF_T16, q, q_len, cache, ext, cache, ext, out, out_len, tq, past, heads, kv_heads,
-                          head_dim, cap, scale, causal);
+                          head_dim, cap, scale, causal, ws, ws_len);
+}
+
+int llmtie_flash_attn_t16(void* stream, const float* q, size_t q_len, const uint16_t* cache, size_t cache_len,
+                          float* out, size_t out_len, size_t tq, size_t past, size_t heads, size_t kv_heads,
+                          size_t head_dim, size_t cap, float scale, int causal) {
+    return llmtie_flash_attn_t16_ws(stream, q, q_len, cache, cache_len, out, out_len, tq, past, heads, kv_heads,
+                                    head_dim, cap, scale, causal, nullptr, 0);
 }
 
 }  // extern "C"

@@ -37,6 +37,11 @@ struct PrefillArgs {
     int xcd, nrb;
     int grid8;  // workgroups of the 1-D launch / 8 (read with the arguments, not from the dispatch packet)
     int cus;          // compute units of the device (set by the entry point)
+    // Split prefill (f16 caches): runs each position block's tiles are cut
+    // into (0 or 1: none) and the caller's workspace, splits * tq * heads *
+    // (hd + 2) floats.
+    int splits;
+    float* ws;
     int light_tiles;  // fast f16 kernel, set by launch_prefill: blocks of at most this many tiles wait first (0: none)
 };
 

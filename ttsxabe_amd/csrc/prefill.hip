@@ -505,29 +505,29 @@ __device__ __forceinline__ void softmax_tile(floatx4 (&sc)[2][2][NQT], int u, in
     l += ps;
 }
 
-// Stores the context rows row0 .. row0 + 15 of head h (query tile u of the
-// wave; rows >= tq skipped) in line order: the wave's O / l goes through its
-// private LDS region R (16 x HD floats, a row's 16-byte chunk c at position
-// c ^ (row & 15), so both the fragment-order writes and the row-order reads
+// Stores columns col0 .. col0 + WD - 1 of the context rows row0 .. row0 + 15
+// (query tile u of the wave; rows >= tq skipped) in line order: the wave's O /
+// l goes through its private LDS region R (16 x WD floats, a row's 16-byte chunk c at position
+// c ^ (row & SW), so both the fragment-order writes and the row-order reads
 // hit 16 different bank groups per 16 lanes), and each store instruction
 // then writes whole lines (LPR lanes a row) instead of 16 rows' half lines
 // (C3 at 512 rows 13.43 -> 13.31 us, at 128 rows 6.28 -> 6.16 us).
-template <int HD, int NQT>
-__device__ __forceinline__ void store_ctx16(float* R, const floatx4 (&o)[HD / 16][NQT], int u, float inv, int lane,
-                                            const PrefillArgs& a, int row0, int h) {
-    constexpr int NT = HD / 16, LPR = HD / 4, RPI = 64 / LPR;
+template <int WD, int NQT>
+__device__ __forceinline__ void store_ctx16(float* R, const floatx4 (&o)[WD / 16][NQT], int u, float inv, int lane,
+                                            const PrefillArgs& a, int row0, int col0) {
+    constexpr int NT = WD / 16, LPR = WD / 4, RPI = 64 / LPR, SW = LPR < 16 ? LPR - 1 : 15;
     const int col = lane & 15, grp = lane >> 4;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         const float4 y = make_float4(o[t][u][0] * inv, o[t][u][1] * inv, o[t][u][2] * inv, o[t][u][3] * inv);
-        *reinterpret_cast<float4*>(R + col * HD + 4 * ((4 * t + grp) ^ col)) = y;
+        *reinterpret_cast<float4*>(R + col * WD + 4 * ((4 * t + grp) ^ (col & SW))) = y;
     }
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         const int row = i * RPI + lane / LPR, c = lane % LPR;
-        const float4 x = *reinterpret_cast<const float4*>(R + row * HD + 4 * (c ^ (row & 15)));
+        const float4 x = *reinterpret_cast<const float4*>(R + row * WD + 4 * (c ^ (row & SW)));
         if (row0 + row < a.tq) {
-            const size_t off = (size_t)(row0 + row) * a.os + (size_t)h * HD + 4 * c;
+            const size_t off = (size_t)(row0 + row) * a.os + (size_t)col0 + 4 * c;
             if (a.out_f16) {
                 half4 y;
                 y[0] = to_h(x.x); y[1] = to_h(x.y); y[2] = to_h(x.z); y[3] = to_h(x.w);
@@ -643,9 +643,14 @@ struct TileLoad {
     }
 };
 
-template <int HD, int KIND, int NQT, int W, bool QL>
+// SPLIT: a launch of few position blocks over many keys (a turn of a long
+// conversation) would leave most of the chip idle behind each block's chain of
+// tiles. The block's tiles are cut into a.splits runs, one workgroup each,
+// which leave (m, l, O) in the caller's workspace for flash_merge_kernel.
+template <int HD, int KIND, int NQT, int W, bool QL, bool SPLIT = false>
 __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(PrefillArgs a) {
     static_assert(W == PW || (W == 8 && KIND == PF_ROWS), "eight waves: encoder rows only");
+    static_assert(!SPLIT || KIND == PF_F16 || KIND == PF_T16, "splits: f16 caches only");
     constexpr int TW = W * LLMTIE_WAVE;
     static_assert(KIND == PF_F16 || KIND == PF_T16 || KIND == PF_F32 || KIND == PF_ROWS, "unknown source");
     // f32 sources (the f32 cache, the stacked encoder rows) are staged through
@@ -670,10 +675,15 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(Prefi
     const int pb = QPW * (W / gb);
     const int group = a.heads / a.kv_heads;
     int rb = blockIdx.x, gy = blockIdx.y;
-    if (a.xcd) {
-        const int item = (int)(blockIdx.x % 8) * a.grid8 + (int)(blockIdx.x / 8);
+    int sp = 0;  // SPLIT: the run of the block's tiles; a head group's runs lie together, row blocks fastest
+    if (SPLIT || a.xcd) {
+        const int item = !SPLIT || a.xcd ? (int)(blockIdx.x % 8) * a.grid8 + (int)(blockIdx.x / 8) : (int)blockIdx.x;
         gy = item / a.nrb;
         rb = item % a.nrb;
+        if constexpr (SPLIT) {
+            sp = gy % a.splits;
+            gy = gy / a.splits;
+        }
     }
     // Causal: heaviest position blocks first.
     const int bx = a.causal ? a.nrb - 1 - rb : rb;
@@ -683,6 +693,13 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(Prefi
     const int p0 = bp0 + (wave / gb) * QPW;
     const int ktot = a.past + a.tq;
     const int kend = a.causal ? min(ktot, a.past + bp0 + pb) : ktot;
+    // The keys this workgroup walks: all below kend, or its run of whole tiles.
+    int kbeg = 0, kstop = kend;
+    if constexpr (SPLIT) {
+        const int nt = (kend + KT - 1) / KT;
+        kbeg = (int)((long)nt * sp / a.splits) * KT;
+        kstop = min(kend, (int)((long)nt * (sp + 1) / a.splits) * KT);
+    }
     // The last key any row of this wave sees, and the last key all of them see.
     const int wlim = a.causal ? min(a.past + p0 + QPW - 1, ktot - 1) : ktot - 1;
     const int wall = a.causal ? min(a.past + p0, ktot - 1) : ktot - 1;
@@ -840,7 +857,7 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(Prefi
         // half the heaviest's tiles) hold their first loads back ~0.85 us so
         // the heavy blocks' queries and first tiles meet less traffic.
         if (a.light_tiles > 0 && (kend + KT - 1) / KT <= a.light_tiles) __builtin_amdgcn_s_sleep(LLMTIE_PF_SLEEP);
-        if (kend > 0) issue(0, t0);
+        if (kbeg < kstop) issue(kbeg, t0);
     }
     const float qsc = a.scale_q ? a.scale : 1.0f;
     half8 qb[NQT][NS];
@@ -998,7 +1015,7 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(Prefi
     auto step = [&](half_t* cur, half_t* nxt, int kv0) __attribute__((always_inline)) {
         __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of `cur` have landed
         __syncthreads();                 // ... and every wave's; `nxt` is free
-        if (kv0 + KT < kend) issue(kv0 + KT, nxt);
+        if (kv0 + KT < kstop) issue(kv0 + KT, nxt);
         if (kv0 + KT > ktot) {
             zero_tail(cur, kv0);
             __syncthreads();
@@ -1039,9 +1056,9 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(Prefi
                 step_staged(jj, JJ % 2 ? t1 : t0, JJ % 2 ? t0 : t1, kv0 + JJ * KT);
             });
     } else {
-        for (int kv0 = 0; kv0 < kend; kv0 += 2 * KT) {
+        for (int kv0 = kbeg; kv0 < kstop; kv0 += 2 * KT) {
             step(t0, t1, kv0);
-            if (kv0 + KT < kend) step(t1, t0, kv0 + KT);
+            if (kv0 + KT < kstop) step(t1, t0, kv0 + KT);
         }
     }
 
@@ -1051,12 +1068,25 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(Prefi
         // before the last tile's barrier, which this wave has passed, and
         // no later tile is issued into it. Wave w's region: 16 x HD floats.
         static_assert(W * 16 * HD * 4 <= (KF + VF) * FH * 2, "the waves' regions fit one tile buffer");
-        const int nt = (kend + KT - 1) / KT;
+        const int nt = (kstop - kbeg + KT - 1) / KT;
         float* R = reinterpret_cast<float*>(nt % 2 ? t1 : t0) + wave * 16 * HD;
 #pragma unroll
         for (int u = 0; u < NQT; ++u) {
             const float lt = sum4grp(l[u]);
-            store_ctx16<HD, NQT>(R, o, u, lt > 0.0f ? 1.0f / lt : 0.0f, lane, a, p0 + 16 * u, h);
+            if constexpr (SPLIT) {
+                // The run's unscaled O laid out as the context is, and each
+                // row's (m, l) behind the runs' contexts.
+                PrefillArgs w = a;
+                w.out = a.ws + (size_t)sp * a.tq * a.os;
+                store_ctx16<HD, NQT>(R, o, u, 1.0f, lane, w, p0 + 16 * u, h * HD);
+                const int r = p0 + 16 * u + col;
+                if (grp == 0 && r < a.tq) {
+                    float2* ml = reinterpret_cast<float2*>(a.ws + (size_t)a.splits * a.tq * a.os);
+                    ml[((size_t)sp * a.tq + r) * a.heads + h] = make_float2(m[u], lt);
+                }
+                continue;
+            }
+            store_ctx16<HD, NQT>(R, o, u, lt > 0.0f ? 1.0f / lt : 0.0f, lane, a, p0 + 16 * u, h * HD);
         }
         return;
     }
@@ -1082,6 +1112,49 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(Prefi
             }
         }
     }
+}
+
+// The context of a split prefill from its runs' (m, l, O): M = max m, O =
+// sum 2^(m - M) O / sum 2^(m - M) l, runs in order, so it does not depend on
+// which ended first. A run that holds no key a row sees has m = PF_NOREF and
+// weight 0. One thread takes four dims of one (row, head); eight runs' loads
+// are in flight at once.
+template <int HD>
+__global__ __launch_bounds__(PT) void flash_merge_kernel(const float* ws, float* out, long rows, int splits) {
+    constexpr int LPR = HD / 4;
+    const long i = (long)blockIdx.x * PT + threadIdx.x;
+    const long row = i / LPR;  // row * heads + head
+    if (row >= rows) return;
+    const float4* o = reinterpret_cast<const float4*>(ws) + i;
+    const float2* ml = reinterpret_cast<const float2*>(ws + (size_t)splits * rows * HD) + row;
+    constexpr int U = 8;
+    float M = PF_NOREF, l = 0.0f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = 0; s0 < splits; s0 += U) {
+        float2 c[U];
+        float4 x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int s = min(s0 + u, splits - 1);
+            c[u] = ml[(size_t)s * rows];
+            x[u] = o[(size_t)s * rows * LPR];
+        }
+        float mn = M;
+#pragma unroll
+        for (int u = 0; u < U; ++u) mn = fmaxf(mn, c[u].x);
+        const float f = ex2(M - mn);
+        M = mn;
+        l *= f;
+        acc = make_float4(acc.x * f, acc.y * f, acc.z * f, acc.w * f);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float w = s0 + u < splits ? ex2(c[u].x - M) : 0.0f;
+            l += w * c[u].y;
+            acc = make_float4(acc.x + w * x[u].x, acc.y + w * x[u].y, acc.z + w * x[u].z, acc.w + w * x[u].w);
+        }
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    reinterpret_cast<float4*>(out)[i] = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
 }
 
 // ------------------------------------------------------------------------
@@ -1343,6 +1416,26 @@ hipError_t launch_prefill(int hd, int kind, int nqt, const PrefillArgs& a, hipSt
     const unsigned pp_items = (unsigned)((a.tq + pp_rows - 1) / pp_rows) * (unsigned)(a.heads / a.gb);
     const bool pp = fast && (kind == PF_T16 || kind == PF_F16) && !(ppe && !atoi(ppe)) &&
                     ((ppe && atoi(ppe)) || pp_items >= 1024);
+    // Split prefills (llmtie_flash_attn_*_ws): a run of a block's tiles a
+    // workgroup, then the merge. LLMTIE_PREFILL_PP compares the two kernels
+    // that share every bit, so it turns them off.
+    if (a.splits > 1 && nqt == 1 && fast && (kind == PF_T16 || kind == PF_F16) && !ppe) {
+        PrefillArgs b = a;
+        b.nrb = (int)grid.x;
+        const unsigned items = grid.x * grid.y * (unsigned)a.splits;
+        b.xcd = items % 8 == 0 && !(getenv("LLMTIE_PREFILL_XCD") && !atoi(getenv("LLMTIE_PREFILL_XCD")));
+        b.grid8 = (int)(items / 8);
+        const long rows = (long)a.tq * a.heads;
+#define FS(HD, KIND)                                                                                        \
+    if (hd == HD && kind == KIND) {                                                                         \
+        hipLaunchKernelGGL((flash_fwd_kernel<HD, KIND, 1, PW, false, true>), dim3(items), block, 0, st, b); \
+        hipLaunchKernelGGL((flash_merge_kernel<HD>), dim3((unsigned)((rows * (HD / 4) + PT - 1) / PT)),     \
+                           dim3(PT), 0, st, a.ws, static_cast<float*>(a.out), rows, a.splits);             \
+        return hipGetLastError();                                                                           \
+    }
+        FS(64, PF_F16) FS(128, PF_F16) FS(64, PF_T16) FS(128, PF_T16)
+#undef FS
+    }
     if (pp) {
         PrefillArgs b = a;
         b.nrb = (a.tq + pp_rows - 1) / pp_rows;

@@ -237,14 +237,24 @@ class Gpu:
     def supports_flash(self, head_dim: int, heads: int, kv_heads: int) -> bool:
         return bool(self._L.llmtie_supports_flash(head_dim, heads, kv_heads))
 
-    def _flash(self, fn, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale, causal, kdt):
+    def _flash(self, fn, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale, causal, kdt, *ws):
         _need(q, _F32, "q")
         _need(k, kdt, "k")
         _need(v, kdt, "v")
         out = torch.empty(max(tq * heads * head_dim, 1), dtype=torch.float32, device=self.device)
         _check(fn(self._stream(), _p(q), _n(q), _p(k), _n(k), _p(v), _n(v), _p(out), tq * heads * head_dim, tq, past,
-                  heads, kv_heads, head_dim, cap, scale, int(bool(causal))))
+                  heads, kv_heads, head_dim, cap, scale, int(bool(causal)), *ws))
         return out[: tq * heads * head_dim]
+
+    def _flash_ws(self, tq, past, heads, kv_heads, head_dim):
+        """The workspace of a prefill off an f16 cache (None: it needs none). It
+        is a torch allocation of the current stream like the output, so the
+        allocator keeps its memory from other streams until the launches on
+        this one are done."""
+        if past + tq <= 512 or min(tq, past, heads, kv_heads, head_dim) < 0:
+            return None  # too few keys to split, or refused by the call itself
+        n = self._L.llmtie_flash_attn_workspace(tq, past, heads, kv_heads, head_dim)
+        return torch.empty(n, dtype=torch.float32, device=self.device) if n else None
 
     def flash_attn(self, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale, causal):
         """device.rs:5702."""
@@ -253,8 +263,9 @@ class Gpu:
 
     def flash_attn_f16(self, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale, causal):
         """device.rs:5754. k, v: f16 caches (float16 or 16-bit integer bits)."""
-        return self._flash(self._L.llmtie_flash_attn_f16, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale,
-                           causal, _H16)
+        ws = self._flash_ws(tq, past, heads, kv_heads, head_dim)
+        return self._flash(self._L.llmtie_flash_attn_f16_ws, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale,
+                           causal, _H16, _p(ws), _n(ws))
 
     def flash_attn_rows(self, qkv, t, heads, head_dim, scale):
         """device.rs:5812. Returns the f16 context [t * heads * head_dim]."""
@@ -383,9 +394,10 @@ class Gpu:
         _need(q, _F32, "q")
         n = tq * heads * cache.head_dim
         out = torch.empty(max(n, 1), dtype=torch.float32, device=self.device)
-        _check(self._L.llmtie_flash_attn_t16(self._stream(), _p(q), _n(q), _p(cache.data), _n(cache.data), _p(out),
-                                             n, tq, past, heads, cache.kv_heads, cache.head_dim, cache.cap,
-                                             scale, int(bool(causal))))
+        ws = self._flash_ws(tq, past, heads, cache.kv_heads, cache.head_dim)
+        _check(self._L.llmtie_flash_attn_t16_ws(self._stream(), _p(q), _n(q), _p(cache.data), _n(cache.data), _p(out),
+                                                n, tq, past, heads, cache.kv_heads, cache.head_dim, cache.cap,
+                                                scale, int(bool(causal)), _p(ws), _n(ws)))
         return out[:n]
 
     def t16_append(self, src, src_off, cache: TiledCache16, n, past, value):
