@@ -39,7 +39,7 @@ def vslot(d, c):
 
 
 def issue_k(hd, f, lane):
-    """(key, chunk) that lane `lane` of K instruction f loads (pfl_issue)."""
+    """(key, chunk) that lane `lane` of K instruction f loads (TileLoad)."""
     cr = hd // 8
     kpi = 64 // cr
     k = f * kpi + lane // cr

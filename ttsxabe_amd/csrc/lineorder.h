@@ -39,24 +39,6 @@ __device__ __forceinline__ int pfl_kslot(int k, int c) {
 }
 // 16-byte slot of chunk c (tile keys 8c .. 8c + 7) of dim d in the V area.
 __device__ __forceinline__ int pfl_vslot(int d, int c) { return (d >> 3) * 64 + (d & 7) * 8 + (c ^ pfl_vsw(d)); }
-// One line-order load instruction of a reference-layout tile at kv0:
-// fragment index f < KF is K, else V (see above).
-template <int HD, int KF>
-__device__ __forceinline__ void pfl_issue(const half_t* kc, __amdgpu_buffer_rsrc_t rv, int f, int lane, size_t kh,
-                                          size_t cap, int kv0, int ktot, half_t* l) {
-    constexpr int CR = HD / 8, KPI = 64 / CR;
-    if (f < KF) {
-        const int k = f * KPI + lane / CR;
-        const int c = (lane % CR) ^ pfl_ksw<HD>(k);
-        const int key = min(kv0 + k, ktot - 1);
-        __builtin_amdgcn_global_load_lds(kc + (kh * cap + key) * HD + 8 * c, l, 16, 0, 0);
-    } else {
-        const int d = 8 * (f - KF) + (lane >> 3);
-        const int c = (lane & 7) ^ pfl_vsw(d);
-        const uint32_t off = (uint32_t)(((kh * HD + d) * cap + kv0 + 8 * c) * 2);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, l, 16, off, 0, 0, 0);
-    }
-}
 // Zero the V entries of keys >= ktot in the tile at kv0 (line order when LO,
 // else fragment order), threads tid, tid + nt, ... over the V area.
 template <int HD, bool LO>

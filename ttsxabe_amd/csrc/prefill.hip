@@ -540,105 +540,91 @@ __device__ __forceinline__ void store_ctx16(float* R, const floatx4 (&o)[WD / 16
 }
 
 // One 64-key tile of an f16 cache into LDS by direct-to-LDS loads, W waves
-// taking fragments wave, wave + W, .. For a tile whose keys are all live, a
-// load's address is a per-lane byte offset fixed for the launch plus a scalar
-// one, from a buffer resource on the tile, so the tile costs each wave its
-// loads and a few scalar instructions: addresses formed per load and per lane
-// were 45 of the 105 vector instructions a tile cost a wave of one query
-// tile, and with two waves a SIMD those kernels are bound by vector issue. The
-// tile that reaches past the keys takes the clamped per-lane addresses (no
-// fixed-offset load relies on a bound). Reference layout, 8192 / 2048 / 512
-// rows of 32/8/128: 557-573 -> 545-559, 58.7 -> 57, 13.7 -> 13.4 us; the tiled
-// cache within 1 % of that.
+// taking fragments wave, wave + W, .. A load's address is a per-lane byte
+// offset fixed for the launch (the tiled cache: plus a scalar one) from a buffer
+// resource on the tile, so a tile costs each wave its loads and a few scalar
+// instructions, by one path for every tile: addresses formed per load and per
+// lane were 45 of the 105 vector instructions a tile cost a wave of one query
+// tile, and a second path for the tile at the end of the keys cost the short
+// launches what the first gained. Where the tile reaches past the keys:
+//   PF_T16: both its halves come from its first block when that is the last
+//     one a row sees, so every address lies in a live block;
+//   PF_F16: K rows up to the capacity are read as they lie and rows past it,
+//     like V past the allocation, are out of the resource's range (every
+//     offset is in the lane's, which the range check covers): zeros.
+// Those scores are masked and V past ktot is zeroed in LDS.
+// 32/8/128 causal, before -> this: tiled cache, 8192 / 1999 / 512 / 128 rows
+// 539 -> 525, 54.2 -> 50.5, 13.2 -> 12.4, 6.7 -> 6.2 us; reference layout, 8192
+// / 2048 / 1024 / 512 rows 542 -> 527, 58 -> 54, 24.6 -> 22.6, 14.2 -> 13.1 us.
 template <int HD, int KIND, int W>
 struct TileLoad {
     static constexpr int NS = HD / 32, NT = HD / 16, KF = 4 * NS, VF = 2 * NT, FH = 64 * 8;
     static constexpr int KI = KF / W, VI = VF / W;  // K and V loads of a wave
     static constexpr int KFB = KF / 2;              // K (and V) fragments of a 32-key block
     static constexpr uint32_t BLK = 128 * HD;       // bytes of a tiled block
+    static constexpr int NO = KIND == PF_T16 ? 1 : KI + VI;
     static_assert(KF % W == 0 && VF % W == 0 && (KFB % W == 0 || W == 2 * KFB), "a wave's fragments are W apart");
 
     const half_t* kc;
-    size_t hb;        // PF_T16: the head's first block; PF_F16: the kv head
-    size_t cap;
+    size_t hb;           // PF_T16: the head's first block; PF_F16: the kv head
+    int cap;
     const char* v;
     uint32_t v_bytes;
-    int lane, wave, w0;  // w0: the wave, as a scalar
-    int ktot, lastb;     // lastb: PF_T16, the last block holding a key some row sees
-    uint32_t ko[2], vo;  // lane offsets (K: of even and odd loads)
-    uint32_t vrow;       // PF_F16: bytes from one V load's dims to the next one's
+    int w0;              // the wave, as a scalar
+    int lastb;           // PF_T16: the last block holding a key some row sees
+    uint32_t off[NO];    // lane offsets (PF_F16: of each load)
 
-    // Byte offset of fragment f in the tile's two tiled blocks.
-    static __device__ __forceinline__ uint32_t t16_off(int f) {
-        const int v = f >= KF, g = v ? f - KF : f;
-        return (uint32_t)(g / KFB) * BLK + v * 64u * HD + (uint32_t)(g % KFB) * 1024u;
-    }
-
-    __device__ __forceinline__ TileLoad(const PrefillArgs& a, int kh, int lane_, int wave_, int ktot_, int kend)
+    __device__ __forceinline__ TileLoad(const PrefillArgs& a, int kh, int lane, int wave, int kend)
         : kc(static_cast<const half_t*>(a.k)),
           hb(KIND == PF_T16 ? (size_t)kh * tiled_nblk(a.cap) : (size_t)kh),
-          cap((size_t)a.cap),
+          cap(a.cap),
           v(static_cast<const char*>(a.v)),
           v_bytes((uint32_t)a.v_bytes),
-          lane(lane_),
-          wave(wave_),
-          w0(__builtin_amdgcn_readfirstlane(wave_)),
-          ktot(ktot_),
+          w0(__builtin_amdgcn_readfirstlane(wave)),
           lastb((max(kend, 1) - 1) >> 5) {
         if constexpr (KIND == PF_T16) {
-            ko[0] = ko[1] = vo = 16u * lane + t16_off(wave);
-            vrow = 0;
+            off[0] = 16u * lane + 1024u * (wave % KFB);
         } else {
             constexpr int CR = HD / 8, KPI = 64 / CR;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int k = (wave + W * j) * KPI + lane / CR;
-                ko[j] = (uint32_t)(k - W * j * KPI) * (2 * HD) + 16u * ((lane % CR) ^ pfl_ksw<HD>(k));
+            for (int i = 0; i < KI; ++i) {
+                const int k = (wave + W * i) * KPI + lane / CR;
+                off[i] = (uint32_t)k * (2 * HD) + 16u * ((lane % CR) ^ pfl_ksw<HD>(k));
             }
-            const int d = 8 * wave + (lane >> 3);
-            vo = (uint32_t)d * (uint32_t)cap * 2u + 16u * ((lane & 7) ^ pfl_vsw(d));
-            vrow = (uint32_t)(8 * W) * (uint32_t)cap * 2u;
+#pragma unroll
+            for (int i = 0; i < VI; ++i) {
+                const int d = 8 * (wave + W * i) + (lane >> 3);
+                off[KI + i] = (uint32_t)d * (uint32_t)cap * 2u + 16u * ((lane & 7) ^ pfl_vsw(d));
+            }
         }
     }
 
     __device__ __forceinline__ void operator()(int kv0, half_t* dst) const {
         half_t* l = dst + w0 * FH;
         if constexpr (KIND == PF_T16) {
-            if ((kv0 >> 5) + 1 <= lastb) {
-                const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-                    const_cast<half_t*>(kc) + (hb + (kv0 >> 5)) * (BLK / 2), 0, 2 * (int)BLK, 0x00020000);
-#pragma unroll
-                for (int i = 0; i < KI + VI; ++i)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, l + W * i * FH, 16, ko[0], t16_off(W * i), 0, 0);
-                return;
-            }
+            const int b = kv0 >> 5;
+            const uint32_t second = b + 1 <= lastb ? BLK : 0;
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<half_t*>(kc) + (hb + b) * (BLK / 2), 0, 2 * (int)BLK, 0x00020000);
 #pragma unroll
             for (int i = 0; i < KI + VI; ++i) {
-                const int f = wave + W * i;
-                const int h = f < KF ? f / (2 * NS) : (f - KF) / NT;
-                const int b = min((kv0 >> 5) + h, lastb);
-                const int in = f < KF ? (f % (2 * NS)) * FH : 32 * HD + ((f - KF) % NT) * FH;
-                __builtin_amdgcn_global_load_lds(kc + (hb + b) * (64 * HD) + in + lane * 8, l + W * i * FH, 16, 0, 0);
+                const int f = W * (i < KI ? i : i - KI);  // of its area, for wave 0
+                const int blk = KFB % W == 0 ? f / KFB : w0 / KFB;
+                const uint32_t in = (i < KI ? 0u : 64u * HD) + 1024u * (f % KFB);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, l + W * i * FH, 16, (int)off[0], blk * second + in, 0, 0);
             }
         } else {
-            if (kv0 + KT <= ktot) {
-                const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-                    const_cast<half_t*>(kc) + (hb * cap + kv0) * HD, 0, KT * 2 * HD, 0x00020000);
-                const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-                    const_cast<char*>(v) + (hb * HD * cap + kv0) * 2, 0, -1, 0x00020000);
+            const size_t vb = (hb * HD * cap + kv0) * 2;
+            const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<half_t*>(kc) + (hb * cap + kv0) * HD, 0, min(cap - kv0, KT) * (2 * HD), 0x00020000);
+            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<char*>(v) + vb, 0, (int)(v_bytes - (uint32_t)vb), 0x00020000);
 #pragma unroll
-                for (int i = 0; i < KI; ++i)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, l + W * i * FH, 16, ko[i & 1], W * i * 1024, 0, 0);
+            for (int i = 0; i < KI; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, l + W * i * FH, 16, (int)off[i], 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < VI; ++i)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, l + (KF + W * i) * FH, 16, vo, i * vrow, 0, 0);
-                return;
-            }
-            const __amdgpu_buffer_rsrc_t rv =
-                __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(v), 0, (int)v_bytes, 0x00020000);
-#pragma unroll
-            for (int i = 0; i < KI + VI; ++i)
-                pfl_issue<HD, KF>(kc, rv, wave + W * i, lane, hb, cap, kv0, ktot, l + W * i * FH);
+            for (int i = 0; i < VI; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, l + (KF + W * i) * FH, 16, (int)off[KI + i], 0, 0, 0);
         }
     }
 };
@@ -841,7 +827,7 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(Prefi
         }
     };
 
-    const TileLoad<HD, STAGED ? PF_T16 : KIND, W> issue(a, kh, lane, wave, ktot, kend);  // unused by the staged kinds
+    const TileLoad<HD, STAGED ? PF_T16 : KIND, W> issue(a, kh, lane, wave, kend);  // unused by the staged kinds
 
     // Q as B operands: qb[u][s] holds dims 32s + 8grp + 0..7 of query p0 + 16u + col.
     // The first tile's loads go out before the query's (the query's first
@@ -1220,7 +1206,7 @@ __global__ __launch_bounds__(PPW * LLMTIE_WAVE, 1) void flash_pp_kernel(PrefillA
     const int wall = a.causal ? min(a.past + p0, ktot - 1) : ktot - 1;
     const int ntile = (kend + KT - 1) / KT;
 
-    const TileLoad<HD, KIND, PPW> issue(a, kh, lane, wave, ktot, kend);
+    const TileLoad<HD, KIND, PPW> issue(a, kh, lane, wave, kend);
     auto zero_tail = [&](half_t* tb, int kv0) __attribute__((always_inline)) {
         pf_zero_tail<HD, KIND == PF_F16>(reinterpret_cast<half8*>(tb + KF * FH), kv0, ktot, tid, TPW);
     };
