@@ -218,3 +218,34 @@ def test_one_scratch_serves_alternating_inputs(gpu):
         q, k, v, exact = cases[rep % 2]
         got = down(gpu.attn_decode_f16(q, k, v, heads, kv, hd, tk, cap, 0.11, False, s))
         assert full_scale_err(exact, got) < 2e-5, f"call {rep}"
+
+
+# One split on eight waves: the first context past four blocks, whole and
+# partial last blocks on every wave, one and two blocks a wave, up to where
+# each layout and group splits, and the first that does.
+@pytest.mark.parametrize("heads,kv,hd,lengths", [
+    (8, 2, 128, (129, 160, 211, 256, 257, 288, 289, 384, 385)), (3, 3, 128, (130, 256, 283, 300, 384)),
+    (4, 4, 64, (129, 255, 256, 257, 384, 400, 512, 513)), (8, 2, 64, (161, 256, 300, 384, 385))])
+def test_contexts_of_one_split_on_eight_waves(gpu, heads, kv, hd, lengths):
+    from ttsxabe_amd.gpu import DecodeScratch, TiledCache16
+    cap, n = 520, heads * hd
+    q = oracle.seq(n, 301)
+    k, v = (oracle.through_f16(oracle.seq(kv * cap * hd, 302 + i)) for i in (0, 1))
+    scratch = DecodeScratch()
+    for tk in lengths:
+        kk, vv = k.reshape(kv, cap, hd).copy(), v.reshape(kv, hd, cap).copy()
+        kk[:, tk:], vv[:, :, tk:] = np.nan, np.nan  # never read into the context
+        want = oracle.decode_f64(q, np.nan_to_num(kk).ravel(), np.nan_to_num(vv).ravel(), heads, kv, hd, tk, cap,
+                                   0.088, False)
+        k16, v16 = up_f16(kk.ravel()), up_f16(vv.ravel())
+        got, twin = gpu.attn_decode_f16_q(up(q), k16, v16, heads, kv, hd, tk, cap, 0.088, False, scratch)
+        assert full_scale_err(want, down(got)) < 2e-5, tk
+        codes, scales = twin.parts()
+        block = down(got).reshape(-1, 32)
+        # The scale is the block maximum times the f32 1 / 127, one rounding.
+        assert np.array_equal(scales.numpy(), np.abs(block).max(1) * (np.float32(1.0) / np.float32(127.0)))
+        t = TiledCache16(kv, hd, cap)
+        gpu.t16_from_ref(k16, v16, t, cap)
+        assert full_scale_err(want, down(gpu.attn_decode_t16(up(q), t, heads, tk, 0.088, False, scratch))) < 2e-5, tk
+        assert full_scale_err(want, down(gpu.attn_decode(up(q), up(kk.ravel()), up(vv.ravel()), heads, kv, hd, tk, cap,
+                                                         0.088, False, scratch))) < 2e-5, tk

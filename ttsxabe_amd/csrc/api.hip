@@ -271,9 +271,31 @@ int compute_units() {
     return cus[dev];
 }
 
+// The longest context, in 32-key blocks, that a single-sequence decode keeps
+// in one split, and the waves its workgroups have then. The cross-workgroup
+// merge (three memory round trips, ~3 us) costs more than the parallelism
+// saves on short contexts. Eight waves (from five blocks on) against four, and
+// against splits, in us: 32/8/128 reference layout, 211 keys 8.0 / 8.35, 256
+// keys 8.5 / 8.8, 300 keys 9.25 / 9.9 / 9.1 split; tiled, 300 keys 6.85 / 8.0 /
+// 8.3, 384 keys 7.15 / 7.8 / 7.9, 420 keys 9.0 / - / 8.35; 20/20/64 f32, 224
+// keys 4.25 / 4.61, 448 keys 5.68 / - / 7.04; f16, 400 keys 6.59 / - / 7.20, 512
+// keys 7.07 / - / 7.34; 32/8/64, 384 keys 6.7 / 7.7, 500 keys 8.2 / - / 7.46.
+size_t one_split_blocks(int kind, size_t group, size_t hd) {
+    if (kind == KV_F16 && hd == 128) return 9;  // its line requests set one compute unit's pace
+    return hd == 64 && group == 1 ? 16 : 12;
+}
+int one_split_waves(size_t tk, int kind, size_t group, size_t hd) {
+    if (getenv("LLMTIE_DECODE_WGS") || getenv("LLMTIE_DECODE_NIT")) return 4;
+    // An f32 cache's hi + lo fragments need four waves' registers (the MFMA
+    // fold at head_dim 64 spilled 85 of them at eight).
+    if (kind == KV_F32 && (hd != 64 || group != 1 || getenv("LLMTIE_DECODE_G1_MFMA"))) return 4;
+    return tk > 128 ? 8 : 4;
+}
+
 // Splits of one head: about `target` workgroups over the whole launch, each
-// wave taking whole 32-key blocks, and never more than the merge can hold.
-void plan_decode(size_t tk_max, size_t units, size_t group, int& nit, int& splits) {
+// wave taking whole 32-key blocks, and never more than the merge can hold; one
+// split up to `one_split` blocks.
+void plan_decode(size_t tk_max, size_t units, size_t group, int& nit, int& splits, size_t one_split = 12) {
     const size_t max_splits = std::min<size_t>(DECODE_MAX_SPLITS, DECODE_MAX_SPLIT_ROWS / std::max<size_t>(1, group));
     // Measured on MI355X: a lone sequence decodes fastest over ~256
     // workgroups (C2: 10.99 us at 128, 10.69 at 256, flat beyond; with the
@@ -288,11 +310,7 @@ void plan_decode(size_t tk_max, size_t units, size_t group, int& nit, int& split
     size_t per_wg = (blocks + want - 1) / want;           // 32-key blocks per workgroup
     size_t n = std::max<size_t>(1, (per_wg + 3) / 4);     // per wave
     if (const char* e = getenv("LLMTIE_DECODE_NIT")) n = std::max(1, atoi(e));
-    // A short context is one split: the cross-workgroup merge (three memory
-    // round trips, ~3 us) costs more than the extra parallelism saves below
-    // ~12 blocks per head (measured: 224 keys 9.2 us unsplit vs 12.4 us in
-    // two splits; 512 keys 10.7 us unsplit vs 10.0 us in two).
-    if (blocks <= 12 && !getenv("LLMTIE_DECODE_WGS") && !getenv("LLMTIE_DECODE_NIT")) n = (blocks + 3) / 4;
+    if (blocks <= one_split && !getenv("LLMTIE_DECODE_WGS") && !getenv("LLMTIE_DECODE_NIT")) n = (blocks + 3) / 4;
     size_t span = 4 * n * 32;
     while ((tk_max + span - 1) / span > max_splits) {
         ++n;
@@ -466,7 +484,10 @@ int decode_common(void* stream, int kind, const float* q, size_t q_len, size_t q
     }
     const size_t group = heads / kv_heads;
     int nit, splits;
-    plan_decode(tk, kv_heads, group, nit, splits);
+    plan_decode(tk, kv_heads, group, nit, splits, one_split_blocks(kind, group, hd));
+    const bool one = splits == 1 && (tk + 31) / 32 <= one_split_blocks(kind, group, hd);
+    const int waves = one ? one_split_waves(tk, kind, group, hd) : 4;
+    if (waves == 8) nit = (int)((tk + 255) / 256);
     const size_t mls = ml_stride(splits, group);
     const size_t part = kv_heads * ((size_t)splits * group * hd + mls);
     const long ml_off = (long)(kv_heads * (size_t)splits * group * hd);
@@ -512,6 +533,7 @@ int decode_common(void* stream, int kind, const float* q, size_t q_len, size_t q
     a.score_l2 = (scale_q ? 1.0f : scale) * 1.4426950408889634f;
     a.qscale = scale_q ? scale : 1.0f;
     a.nit = nit;
+    a.waves = waves;
     a.splits = splits;
     a.ml_stride = (long)mls;
     a.two_phase = two_phase_merge(splits, kv_heads);

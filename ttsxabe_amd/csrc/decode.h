@@ -40,6 +40,7 @@ struct DecodeArgs {
     float qscale;            // applied to q before it is split
     int nit;                 // 32-key blocks per wave per split
     int splits;              // grid.x: splits of the longest sequence
+    int waves;               // waves a workgroup: 8 (one split, 5 to 16 blocks), else 4
     int two_phase;           // merge in a second launch (else the last split's workgroup merges)
     // Stream-K batch (sk != 0, Q8_0 cache, nseq <= 64): a 1-D grid of
     // `items` workgroups whose waves each take an equal range of the batch's

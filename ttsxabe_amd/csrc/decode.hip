@@ -951,8 +951,13 @@ __device__ __forceinline__ bool one_xcd(unsigned long long c) {
     return n * s2 == s1 * s1;
 }
 
-template <int HD, int KIND, int VA, bool G1>
-__global__ __launch_bounds__(DT, KIND == KV_F32 ? 1 : 2) void attn_decode_kernel(DecodeArgs a) {
+// W waves a workgroup: 4, or 8 for a context of one split and 5 to 16 blocks
+// (a.waves). There a wave's chain of folds is what the launch waits for, and
+// nothing is handed to another workgroup, so twice the waves halve it (the
+// times stand at the plan's rule, one_split_blocks).
+template <int HD, int KIND, int VA, bool G1, int W = DW>
+__global__ __launch_bounds__(W * LLMTIE_WAVE, KIND == KV_F32 ? 1 : 2) void attn_decode_kernel(DecodeArgs a) {
+    constexpr int DW = W, DT = W * LLMTIE_WAVE;  // this launch's (the merge's are four waves')
     constexpr int NS = HD / 32;
     constexpr int NT = HD / 16;
     constexpr bool TILED = KIND == KV_T16 || KIND == KV_TQ8;
@@ -1195,7 +1200,7 @@ __global__ __launch_bounds__(DT, KIND == KV_F32 ? 1 : 2) void attn_decode_kernel
         ts = a.twin_scales + (oo >> 5);
     }
     const int n = group * HD;
-    if (nsplit == 1) {
+    if (W != llmtie::DW || nsplit == 1) {  // eight waves: one split always
         for (int e = tid; e < n; e += DT) {
             const int g = e / HD, d = e % HD;
             float f[DW];
@@ -2106,6 +2111,11 @@ __global__ __launch_bounds__(DT, 1) void attn_decode_sk_kernel(DecodeArgs a) {
     }
 }
 
+#define DECODE_INST8(HD, KIND, VA, G1) template __global__ void attn_decode_kernel<HD, KIND, VA, G1, 8>(DecodeArgs);
+#define DECODE_INST82(HD, KIND, VA) DECODE_INST8(HD, KIND, VA, false) DECODE_INST8(HD, KIND, VA, true)
+DECODE_INST82(64, KV_F16, 16) DECODE_INST82(128, KV_F16, 16) DECODE_INST82(64, KV_F16, 8) DECODE_INST82(128, KV_F16, 8)
+DECODE_INST82(64, KV_T16, 16) DECODE_INST82(128, KV_T16, 16)
+DECODE_INST8(64, KV_F32, 16, true) DECODE_INST8(64, KV_F32, 8, true)
 #define DECODE_INST(HD, KIND, VA, G1) template __global__ void attn_decode_kernel<HD, KIND, VA, G1>(DecodeArgs);
 #define DECODE_INST2(HD, KIND, VA) DECODE_INST(HD, KIND, VA, false) DECODE_INST(HD, KIND, VA, true)
 DECODE_INST2(64, KV_F16, 16) DECODE_INST2(128, KV_F16, 16) DECODE_INST2(64, KV_F16, 8) DECODE_INST2(128, KV_F16, 8)
@@ -2145,6 +2155,20 @@ static hipError_t launch_attn(int hd, int kind, const DecodeArgs& a, int kv_head
     const int va = (kind == KV_T16 || kind == KV_TQ8) ? 16 : (((long)a.cap * esz) % 16 == 0 ? 16 : 8);
     // Group 1 (MHA) folds on the VALU.
     const bool g1 = a.group == 1 && kind != KV_TQ8 && !getenv("LLMTIE_DECODE_G1_MFMA");
+#define L8(HD, KIND, VA, G1)                                                                                          \
+    if (hd == HD && kind == KIND && va == VA && g1 == G1) {                                                           \
+        hipLaunchKernelGGL((attn_decode_kernel<HD, KIND, VA, G1, 8>), grid, dim3(8 * LLMTIE_WAVE), 0, st, b);         \
+        return hipGetLastError();                                                                                     \
+    }
+#define L82(HD, KIND, VA) L8(HD, KIND, VA, false) L8(HD, KIND, VA, true)
+    if (a.waves == 8) {
+        if (a.splits != 1) return hipErrorInvalidValue;
+        L82(64, KV_F16, 16) L82(128, KV_F16, 16) L82(64, KV_F16, 8) L82(128, KV_F16, 8)
+        L82(64, KV_T16, 16) L82(128, KV_T16, 16) L8(64, KV_F32, 16, true) L8(64, KV_F32, 8, true)
+        return hipErrorInvalidValue;
+    }
+#undef L82
+#undef L8
 #define L(HD, KIND, VA, G1)                                                                    \
     if (hd == HD && kind == KIND && va == VA && g1 == G1) {                                    \
         hipLaunchKernelGGL((attn_decode_kernel<HD, KIND, VA, G1>), grid, block, 0, st, b);      \
