@@ -155,3 +155,19 @@ def test_group_widths(gpu, hd, heads, kv):
     """GQA groups of 16 (the largest query buffers) and 1 (MHA)."""
     tk = (oracle.uniform_int(9, 34 + heads, 1, 700)).astype(np.int32)
     check_batch(gpu, hd, heads, kv, 9, 704, tk, np.arange(9, dtype=np.int32)[::-1].copy(), 44 + heads)
+
+
+# Both launches at batches on either side of the rule between them: one
+# sequence, a split and an unsplit plan, spans of 1024 keys (more than 64 heads
+# over more than one round of workgroups), lengths of one key and of a block's
+# edges.
+@pytest.mark.parametrize("static", ["0", "1", None])
+@pytest.mark.parametrize("hd,heads,kv,lengths", [
+    (128, 32, 8, [2500]), (128, 8, 8, [1, 32, 33, 700, 64]), (64, 16, 4, [1, 31, 900, 320, 257]),
+    (128, 16, 8, [1, 1023, 1024, 1025, 129, 40, 1500, 600, 31, 32, 33, 777])])
+def test_stream_k_and_the_planned_grid_are_the_same_attention(gpu, hd, heads, kv, lengths, static, monkeypatch):
+    if static is not None:
+        monkeypatch.setenv("LLMTIE_DECODE_STATIC", static)
+    n = len(lengths)
+    check_batch(gpu, hd, heads, kv, n, 2528, np.array(lengths, np.int32), np.arange(n, dtype=np.int32)[::-1].copy(),
+                45 + n)

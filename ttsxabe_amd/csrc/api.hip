@@ -320,6 +320,35 @@ void plan_decode(size_t tk_max, size_t units, size_t group, int& nit, int& split
     splits = (int)((tk_max + span - 1) / span);
 }
 
+// Whether a batched Q8_0 decode runs stream-K (one workgroup per compute unit,
+// each wave an equal share of the batch's blocks) rather than on the
+// host-planned grid (splits of the longest sequence), whose plan it may widen.
+// Stream-K balances ragged lengths, but each wave holds a head's pieces, so a
+// batch of few blocks pays for merging hundreds of them: the host only knows
+// the lengths' bound, so the line is drawn at the bytes that it allows. Host
+// plan / stream-K, us, at 8 kv heads of 128: 1 sequence of 4000, 9.2 / 42.8; 4 of
+// 500-2000, 10.3 / 22.7; 8 of 256-4096 (bound 71 MB), 16.4 / 25.6; 8 of
+// 6000-8000 (139 MB), 28 / 36; 32 of 100-1000 (70 MB), 14.2 / 18.3; 12 of
+// 20-8000 (209 MB), 37-44 / 33; 16 of 500-4000 (139 MB), 25-30 / 28; 32 of
+// 256-8192 (570 MB), 71 / 58.8. More than 64 sequences always take the plan.
+bool plan_q8_batch(size_t nseq, size_t kv_heads, size_t hd, size_t max_tk, int& nit, int& splits) {
+    const char* e = getenv("LLMTIE_DECODE_STATIC");
+    if (nseq > 64 || (e && atoi(e))) return false;
+    if (e) return true;
+    const size_t units = nseq * kv_heads;
+    const double mb = (double)units * (double)max_tk * (double)(2 * hd + hd / 8) * 1e-6;
+    if (mb > (units <= 64 ? 150.0 : 75.0)) return true;
+    // Beyond one round of workgroups, spans of 1024 keys (eight blocks a wave):
+    // 12 sequences of 100-1000, 10.8 us against 14.0 in three splits each; 20,
+    // 12.6 / 15.5; 32, 14.2 / 20.9.
+    if (units > 64 && units * (size_t)splits > 256 && nit < 8 && !getenv("LLMTIE_DECODE_NIT") &&
+        !getenv("LLMTIE_DECODE_WGS")) {
+        nit = 8;
+        splits = (int)((max_tk + 1023) / 1024);
+    }
+    return false;
+}
+
 // Whether the split partials are merged by a second launch rather than by
 // the last-arriving workgroup of each head.
 int two_phase_merge(int splits, size_t units) {
@@ -741,10 +770,7 @@ int llmtie_attn_decode_q8_batch(void* stream, const float* q, size_t q_len, cons
     const size_t group = heads / kv_heads;
     int nit, splits;
     plan_decode(max_tk, kv_heads * nseq, group, nit, splits);
-    // Up to 64 sequences go through the stream-K kernel, one workgroup per
-    // compute unit, each wave an equal share of the batch's blocks; a larger
-    // batch through the host-planned grid (splits of the longest sequence).
-    const bool sk = nseq <= 64 && !getenv("LLMTIE_DECODE_STATIC");
+    const bool sk = plan_q8_batch(nseq, kv_heads, head_dim, max_tk, nit, splits);
     const int items = sk ? compute_units() : 0;
     const size_t mls = ml_stride(splits, group);
     size_t part = nseq * kv_heads * ((size_t)splits * group * head_dim + mls);
