@@ -216,7 +216,8 @@ __global__ __launch_bounds__(KB) void append_vt_kernel(const float* src, T* dst,
 // trip and an angle: with the head width known (HD; 0: any) the index
 // arithmetic is shifts, and the row's values are loaded before the angle is
 // evaluated, so the two overlap. 32/8/128 in a graph of launches (a fill of the
-// same size takes 1.85 us): f16 2.46 -> 2.30 us, tiled 2.47 -> 2.34, Q8_0 (its block maxima on DPP, not LDS shuffles) 2.77 -> 2.56.
+// same size takes 1.85 us): f16 2.46 -> 2.30 us, tiled 2.47 -> 2.34, Q8_0 (its
+// block maxima on DPP, not LDS shuffles) 2.77 -> 2.56.
 //
 // The pair of element e of a row of heads, rotated at position p.
 template <int HD>

@@ -229,7 +229,8 @@ class Gpu:
     def _stream(self):
         # The current stream's handle without a Stream object: a call of a few
         # launches is as long as its host work (three calls of the f32 prompt
-        # layer took 25.2 us of host work with the ctypes and Stream objects, 17.2 us without).
+        # layer took 25.2 us of it with the ctypes and Stream objects, 17.2 us
+        # without).
         return torch._C._cuda_getCurrentRawStream(self.device.index)
 
     # ------------------------------------------------------------- prefill
