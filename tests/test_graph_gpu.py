@@ -125,3 +125,35 @@ def test_scratch_growth_keeps_an_earlier_graph_valid(gpu):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(eager[0], outs[0]), f"replay {i} after growth differs"
+
+
+def test_one_batch_sizes_the_scratch_for_every_batch_as_wide(gpu):
+    """A batch of short sequences runs on the host-planned grid, one of long
+    sequences on stream-K: the first leaves a scratch that the second can be
+    captured with, and the other way round."""
+    from tests.test_q8_decode_gpu import load, random_q8_cache
+    from ttsxabe_amd.gpu import DecodeScratch, KvCacheQ8
+    heads, kv, hd, slots, cap = 32, 8, 128, 16, 4096
+    cache = KvCacheQ8(slots, kv, hd, cap)
+    load(cache, *random_q8_cache(slots, kv, hd, cap, 77))
+    q = up(oracle.normal(slots * heads * hd, 78))
+    slot = up(np.arange(slots, dtype=np.int32), torch.int32)
+    tks = {n: up(oracle.uniform_int(slots, 79, 1, n).astype(np.int32), torch.int32) for n in (100, 4000)}
+    for first, then in ((100, 4000), (4000, 100)):
+        run = lambda n, s: gpu.attn_decode_q8_batch(q, cache, tks[n], slot, n, heads, 0.088, False, s)
+        want = run(then, DecodeScratch()).clone()
+        st = torch.cuda.Stream()
+        st.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(st):
+            s = DecodeScratch()
+            run(first, s)
+            torch.cuda.synchronize()
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=st):
+                out = run(then, s)
+        torch.cuda.synchronize()
+        for _ in range(3):
+            out.fill_(float("nan"))
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), (first, then)

@@ -770,15 +770,23 @@ int llmtie_attn_decode_q8_batch(void* stream, const float* q, size_t q_len, cons
     const size_t group = heads / kv_heads;
     int nit, splits;
     plan_decode(max_tk, kv_heads * nseq, group, nit, splits);
-    const bool sk = plan_q8_batch(nseq, kv_heads, head_dim, max_tk, nit, splits);
-    const int items = sk ? compute_units() : 0;
+    bool sk = plan_q8_batch(nseq, kv_heads, head_dim, max_tk, nit, splits);
     const size_t mls = ml_stride(splits, group);
     size_t part = nseq * kv_heads * ((size_t)splits * group * head_dim + mls);
     long ml_off = (long)(nseq * kv_heads * (size_t)splits * group * head_dim);
+    const size_t slots2 = (size_t)compute_units() * SK_WAVES * 2;
+    const size_t sk_part = slots2 * (16 * head_dim + 32);
+    // Every batch of up to 64 sequences takes the partials of the stream-K
+    // slots, whichever grid it runs on, so that a scratch which served one of
+    // them serves the next under capture, whatever its lengths' bound.
+    if (nseq <= 64 && !getenv("LLMTIE_DECODE_STATIC")) {
+        sk = sk || part > sk_part;
+        part = sk_part;
+    }
+    const int items = sk ? compute_units() : 0;
     if (sk) {
-        const size_t slots2 = (size_t)items * SK_WAVES * 2;
         ml_off = (long)(slots2 * 16 * head_dim);
-        part = slots2 * (16 * head_dim + 32);
+        part = sk_part;
     }
     int r = ensure_scratch(scratch, part, nseq * kv_heads * CTR_STRIDE, S(stream));
     if (r != LLMTIE_OK) return r;
