@@ -249,3 +249,36 @@ def test_contexts_of_one_split_on_eight_waves(gpu, heads, kv, hd, lengths):
         assert full_scale_err(want, down(gpu.attn_decode_t16(up(q), t, heads, tk, 0.088, False, scratch))) < 2e-5, tk
         assert full_scale_err(want, down(gpu.attn_decode(up(q), up(kk.ravel()), up(vv.ravel()), heads, kv, hd, tk, cap,
                                                          0.088, False, scratch))) < 2e-5, tk
+
+
+def test_a_split_that_the_scratch_has_no_room_for_is_one_split(gpu):
+    """310 reference-layout keys of head_dim 128 run in splits, but in one
+    where the partials have no room: a scratch that only a short context
+    sized, under capture, and more kv heads of 16 query heads than the fixed
+    scratch takes splits of."""
+    from ttsxabe_amd.gpu import DecodeScratch
+    hd, tk, cap = 128, 310, 312
+    for heads, kv in ((32, 8), (4096, 256)):
+        q = up(oracle.seq(heads * hd, 61))
+        k, v = up_f16(oracle.seq(kv * cap * hd, 62)), up_f16(oracle.seq(kv * cap * hd, 63))
+        scale = hd ** -0.5
+        if kv == 256:
+            got = gpu.attn_decode_f16_noalloc(q, k, v, heads, kv, hd, tk, cap, scale, False)
+        else:
+            st = torch.cuda.Stream()
+            st.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(st):
+                s = DecodeScratch()
+                gpu.attn_decode_f16(q, k, v, heads, kv, hd, 40, cap, scale, False, s)
+                torch.cuda.synchronize()
+                g = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(g, stream=st):
+                    got = gpu.attn_decode_f16(q, k, v, heads, kv, hd, tk, cap, scale, False, s)
+            for _ in range(2):
+                got.fill_(float("nan"))
+                g.replay()
+                torch.cuda.synchronize()
+        exact = oracle.decode_f64(oracle.seq(heads * hd, 61), oracle.through_f16(oracle.seq(kv * cap * hd, 62)),
+                                  oracle.through_f16(oracle.seq(kv * cap * hd, 63)), heads, kv, hd, tk, cap, scale,
+                                  False)
+        assert np.abs(exact - down(got)).max() / np.abs(exact).max() < 2e-5, (heads, kv)

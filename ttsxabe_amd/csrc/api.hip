@@ -513,8 +513,23 @@ int decode_common(void* stream, int kind, const float* q, size_t q_len, size_t q
     }
     const size_t group = heads / kv_heads;
     int nit, splits;
-    plan_decode(tk, kv_heads, group, nit, splits, one_split_blocks(kind, group, hd));
-    const bool one = splits == 1 && (tk + 31) / 32 <= one_split_blocks(kind, group, hd);
+    size_t one_split = one_split_blocks(kind, group, hd);
+    plan_decode(tk, kv_heads, group, nit, splits, one_split);
+    // Contexts of up to 12 blocks that a cache kind splits for speed stay in
+    // one split where the partials of several have no room: beyond the fixed
+    // scratch, or under capture with a scratch that has to grow first.
+    if (splits > 1 && one_split < 12 && (tk + 31) / 32 <= 12) {
+        const size_t want = kv_heads * ((size_t)splits * group * hd + ml_stride(splits, group));
+        bool room = noalloc ? want <= NOALLOC_PART_FLOATS : scratch->part_cap >= want;
+        if (!noalloc && !room) {
+            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+            const hipError_t e = hipStreamIsCapturing(S(stream), &cs);
+            if (e != hipSuccess) return driver("hipStreamIsCapturing", e);
+            room = cs == hipStreamCaptureStatusNone;
+        }
+        if (!room) plan_decode(tk, kv_heads, group, nit, splits, one_split = 12);
+    }
+    const bool one = splits == 1 && (tk + 31) / 32 <= one_split;
     const int waves = one ? one_split_waves(tk, kind, group, hd) : 4;
     if (waves == 8) nit = (int)((tk + 255) / 256);
     const size_t mls = ml_stride(splits, group);
