@@ -207,3 +207,18 @@ def test_the_prefill_workspace_is_asked_for_where_keys_outnumber_rows():
         assert need(*shape) == 0, shape
     # Never more than about 800 workgroups' 64 rows of partials.
     assert max(need(t, p, 32, 8, 128) for t in range(1, 700, 13) for p in range(0, 8000, 533)) <= 800 * 64 * 130
+
+
+def test_a_prefill_without_memory_for_its_workspace_is_not_split(monkeypatch):
+    """A full card refuses the workspace, not the call."""
+    import torch
+    from ttsxabe_amd.gpu import Gpu
+    g = Gpu.__new__(Gpu)
+    g._L, g.device = _lib.lib(), torch.device("cpu")
+    assert g._flash_ws(173, 3011, 32, 8, 128).numel() == _lib.lib().llmtie_flash_attn_workspace(173, 3011, 32, 8, 128) > 0
+
+    def full(*a, **k):
+        raise torch.OutOfMemoryError("out of memory")
+
+    monkeypatch.setattr(torch, "empty", full)
+    assert g._flash_ws(173, 3011, 32, 8, 128) is None

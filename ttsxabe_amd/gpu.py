@@ -255,7 +255,12 @@ class Gpu:
         if past + tq <= 512 or min(tq, past, heads, kv_heads, head_dim) < 0:
             return None  # too few keys to split, or refused by the call itself
         n = self._L.llmtie_flash_attn_workspace(tq, past, heads, kv_heads, head_dim)
-        return torch.empty(n, dtype=torch.float32, device=self.device) if n else None
+        if not n:
+            return None
+        try:
+            return torch.empty(n, dtype=torch.float32, device=self.device)
+        except torch.OutOfMemoryError:
+            return None  # the unsplit prefill needs nothing beside its output
 
     def flash_attn(self, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale, causal):
         """device.rs:5702."""
