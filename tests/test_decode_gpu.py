@@ -251,34 +251,35 @@ def test_contexts_of_one_split_on_eight_waves(gpu, heads, kv, hd, lengths):
                                                          0.088, False, scratch))) < 2e-5, tk
 
 
-def test_a_split_that_the_scratch_has_no_room_for_is_one_split(gpu):
-    """310 reference-layout keys of head_dim 128 run in splits, but in one
-    where the partials have no room: a scratch that only a short context
-    sized, under capture, and more kv heads of 16 query heads than the fixed
-    scratch takes splits of."""
+# Reference-layout contexts around the line between one split and several. A
+# scratch that only a short context sized (of as many heads, and of others
+# whose one split takes as much), under capture; and, for 256 kv heads of 16
+# query heads, partials of several splits past the fixed scratch.
+@pytest.mark.parametrize("heads,kv,tk,warm", [
+    (32, 8, 288, (32, 8)), (32, 8, 289, (32, 8)), (32, 8, 384, (32, 8)), (40, 40, 384, (40, 40)),
+    (28, 4, 310, (20, 20)), (4096, 256, 310, (4096, 256))])
+def test_one_call_has_one_result_whatever_room_its_scratch_has(gpu, heads, kv, tk, warm):
     from ttsxabe_amd.gpu import DecodeScratch
-    hd, tk, cap = 128, 310, 312
-    for heads, kv in ((32, 8), (4096, 256)):
-        q = up(oracle.seq(heads * hd, 61))
-        k, v = up_f16(oracle.seq(kv * cap * hd, 62)), up_f16(oracle.seq(kv * cap * hd, 63))
-        scale = hd ** -0.5
-        if kv == 256:
-            got = gpu.attn_decode_f16_noalloc(q, k, v, heads, kv, hd, tk, cap, scale, False)
-        else:
-            st = torch.cuda.Stream()
-            st.wait_stream(torch.cuda.current_stream())
-            with torch.cuda.stream(st):
-                s = DecodeScratch()
-                gpu.attn_decode_f16(q, k, v, heads, kv, hd, 40, cap, scale, False, s)
-                torch.cuda.synchronize()
-                g = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(g, stream=st):
-                    got = gpu.attn_decode_f16(q, k, v, heads, kv, hd, tk, cap, scale, False, s)
-            for _ in range(2):
-                got.fill_(float("nan"))
-                g.replay()
-                torch.cuda.synchronize()
-        exact = oracle.decode_f64(oracle.seq(heads * hd, 61), oracle.through_f16(oracle.seq(kv * cap * hd, 62)),
-                                  oracle.through_f16(oracle.seq(kv * cap * hd, 63)), heads, kv, hd, tk, cap, scale,
-                                  False)
-        assert np.abs(exact - down(got)).max() / np.abs(exact).max() < 2e-5, (heads, kv)
+    hd, cap, scale = 128, 384, 128 ** -0.5
+    q, k, v = (oracle.seq(n, 61 + i) for i, n in enumerate((heads * hd, kv * cap * hd, kv * cap * hd)))
+    dq, dk, dv = up(q), up_f16(k), up_f16(v)
+    call = lambda s: gpu.attn_decode_f16(dq, dk, dv, heads, kv, hd, tk, cap, scale, False, s)
+    want = call(DecodeScratch())
+    assert torch.equal(gpu.attn_decode_f16_noalloc(dq, dk, dv, heads, kv, hd, tk, cap, scale, False), want)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(st):
+        s = DecodeScratch()
+        gpu.attn_decode_f16(dq, up_f16(np.zeros(warm[1] * 40 * hd)), up_f16(np.zeros(warm[1] * 40 * hd)), *warm, hd,
+                            40, 40, scale, False, s)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            got = call(s)
+    for _ in range(2):
+        got.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+    exact = oracle.decode_f64(q, oracle.through_f16(k), oracle.through_f16(v), heads, kv, hd, tk, cap, scale, False)
+    assert np.abs(exact - down(want)).max() / np.abs(exact).max() < 2e-5

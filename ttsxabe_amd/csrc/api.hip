@@ -271,17 +271,35 @@ int compute_units() {
     return cus[dev];
 }
 
+// Floats of the (m, l) area per (sequence, kv head): whole 256-byte lines,
+// so no line is shared by two heads' partials.
+size_t ml_stride(int splits, size_t group) { return ((size_t)splits * group * 2 + 63) / 64 * 64; }
+
+// Sizes of the no-allocation decode's fixed scratch: split partials, then
+// arrival counters (CTR_STRIDE words per kv head).
+constexpr size_t NOALLOC_PART_FLOATS = (size_t)1 << 20;
+constexpr size_t NOALLOC_CTR_WORDS = (size_t)256 * CTR_STRIDE;
+
 // The longest context, in 32-key blocks, that a single-sequence decode keeps
 // in one split, and the waves its workgroups have then. The cross-workgroup
 // merge (three memory round trips, ~3 us) costs more than the parallelism
 // saves on short contexts. Eight waves (from five blocks on) against four, and
 // against splits, in us: 32/8/128 reference layout, 211 keys 8.0 / 8.35, 256
-// keys 8.5 / 8.8, 300 keys 9.25 / 9.9 / 9.1 split; tiled, 300 keys 6.85 / 8.0 /
-// 8.3, 384 keys 7.15 / 7.8 / 7.9, 420 keys 9.0 / - / 8.35; 20/20/64 f32, 224
-// keys 4.25 / 4.61, 448 keys 5.68 / - / 7.04; f16, 400 keys 6.59 / - / 7.20, 512
-// keys 7.07 / - / 7.34; 32/8/64, 384 keys 6.7 / 7.7, 500 keys 8.2 / - / 7.46.
-size_t one_split_blocks(int kind, size_t group, size_t hd) {
-    if (kind == KV_F16 && hd == 128) return 9;  // its line requests set one compute unit's pace
+// keys 8.5 / 8.8; tiled, 300 keys 6.85 / 8.0 / 8.3, 384 keys 7.15 / 7.8 / 7.9,
+// 420 keys 9.0 / - / 8.35; 20/20/64 f32, 224 keys 4.25 / 4.61, 448 keys 5.68 /
+// - / 7.04; f16, 400 keys 6.59 / - / 7.20, 512 keys 7.07 / - / 7.34; 32/8/64,
+// 384 keys 6.7 / 7.7, 500 keys 8.2 / - / 7.46.
+// The reference layout at head_dim 128 splits from ten blocks on (its line
+// requests set one compute unit's pace): 300 / 320 / 352 / 384 keys, three
+// splits against one: 32/8, 9.36 9.31 9.35 9.18 / 9.88 9.80 10.2 10.5; 16/8,
+// 9.23 9.20 9.20 9.24 / 9.70 9.63 10.2 10.8; 8/2, 8.96 8.72 8.78 8.57 / 9.50
+// 8.89 9.39 9.97; 40/40, 8.68 8.68 8.69 8.70 / 8.61 8.39 8.68 9.11. The line
+// lies by the shape alone, so that a call has one result whatever scratch it
+// is given: not where three splits' partials pass the fixed scratch, and every
+// growing scratch has room for them (ensure_scratch).
+size_t one_split_blocks(int kind, size_t kv_heads, size_t group, size_t hd) {
+    if (kind == KV_F16 && hd == 128 && kv_heads * (3 * group * hd + ml_stride(3, group)) <= NOALLOC_PART_FLOATS)
+        return 9;
     return hd == 64 && group == 1 ? 16 : 12;
 }
 int one_split_waves(size_t tk, int kind, size_t group, size_t hd) {
@@ -360,10 +378,6 @@ int two_phase_merge(int splits, size_t units) {
     return (size_t)splits * units > 1024 ? 1 : 0;
 }
 
-// Floats of the (m, l) area per (sequence, kv head): whole 256-byte lines,
-// so no line is shared by two heads' partials.
-size_t ml_stride(int splits, size_t group) { return ((size_t)splits * group * 2 + 63) / 64 * 64; }
-
 // Whether a host-planned in-launch merge keeps every head on one XCD: the
 // dispatcher deals a launch's workgroups to the eight XCDs of gfx950 in
 // turn, so workgroups L and L + 8k share an XCD (which XCD a launch starts on
@@ -424,6 +438,10 @@ int ensure_scratch(llmtie_decode_scratch* s, size_t part_floats, size_t ctrs, hi
     if (s->part_cap < part_floats) {
         size_t want = 1024;
         while (want < part_floats) want <<= 1;
+        // Room for three splits' partials of any decode whose one split fits:
+        // a context of ten to twelve blocks may be captured after a shorter
+        // one sized the scratch (one_split_blocks).
+        want = std::max(want, std::min(4 * want, NOALLOC_PART_FLOATS));
         float* p = nullptr;
         e = hipMalloc(&p, want * sizeof(float));
         if (e != hipSuccess) return driver("allocating", e);
@@ -462,10 +480,6 @@ struct FixedScratch {
     size_t ctr_cap;   // words
 };
 
-// Sizes of the no-allocation decode's fixed scratch: split partials, then
-// arrival counters (CTR_STRIDE words per kv head).
-constexpr size_t NOALLOC_PART_FLOATS = (size_t)1 << 20;
-constexpr size_t NOALLOC_CTR_WORDS = (size_t)256 * CTR_STRIDE;
 int noalloc_scratch(hipStream_t st, FixedScratch& f);
 
 // The checks and the launch behind every single-sequence decode
@@ -513,22 +527,8 @@ int decode_common(void* stream, int kind, const float* q, size_t q_len, size_t q
     }
     const size_t group = heads / kv_heads;
     int nit, splits;
-    size_t one_split = one_split_blocks(kind, group, hd);
+    const size_t one_split = one_split_blocks(kind, kv_heads, group, hd);
     plan_decode(tk, kv_heads, group, nit, splits, one_split);
-    // Contexts of up to 12 blocks that a cache kind splits for speed stay in
-    // one split where the partials of several have no room: beyond the fixed
-    // scratch, or under capture with a scratch that has to grow first.
-    if (splits > 1 && one_split < 12 && (tk + 31) / 32 <= 12) {
-        const size_t want = kv_heads * ((size_t)splits * group * hd + ml_stride(splits, group));
-        bool room = noalloc ? want <= NOALLOC_PART_FLOATS : scratch->part_cap >= want;
-        if (!noalloc && !room) {
-            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-            const hipError_t e = hipStreamIsCapturing(S(stream), &cs);
-            if (e != hipSuccess) return driver("hipStreamIsCapturing", e);
-            room = cs == hipStreamCaptureStatusNone;
-        }
-        if (!room) plan_decode(tk, kv_heads, group, nit, splits, one_split = 12);
-    }
     const bool one = splits == 1 && (tk + 31) / 32 <= one_split;
     const int waves = one ? one_split_waves(tk, kind, group, hd) : 4;
     if (waves == 8) nit = (int)((tk + 255) / 256);
