@@ -157,3 +157,35 @@ def test_one_batch_sizes_the_scratch_for_every_batch_as_wide(gpu):
             g.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, want), (first, then)
+
+
+@pytest.mark.parametrize("f16", [False, True])
+def test_an_eager_step_of_an_unsplit_context_sizes_the_scratch_for_the_next(gpu, f16):
+    """Multi-head contexts of up to 512 keys at head_dim 64 run in one split,
+    longer ones in several: a step on either side leaves a scratch that the
+    longer one can be captured with, also where the shorter one's own partials
+    fit what the scratch already holds."""
+    from ttsxabe_amd.gpu import DecodeScratch
+    heads, hd, cap = 128, 64, 640
+    q, k, v = (oracle.seq(n, 91 + i) for i, n in enumerate((heads * hd, heads * cap * hd, heads * cap * hd)))
+    load = up_f16 if f16 else up
+    dq, dk, dv = up(q), load(k), load(v)
+    fn = gpu.attn_decode_f16 if f16 else gpu.attn_decode
+    step = lambda h, tk, s: fn(dq[: h * hd], dk[: h * cap * hd], dv[: h * cap * hd], h, h, hd, tk, cap, 0.125, True, s)
+    want = step(heads, 600, DecodeScratch()).clone()
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(st):
+        s = DecodeScratch()
+        step(32, 40, s)
+        step(heads, 500, s)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            out = step(heads, 600, s)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)

@@ -402,23 +402,27 @@ int retire(llmtie_decode_scratch* s, void* p) {
     return LLMTIE_OK;
 }
 
-int ensure_scratch(llmtie_decode_scratch* s, size_t part_floats, size_t ctrs, hipStream_t st) {
+// `room`: partial floats an eager call makes room for beyond its own, so that
+// a longer context may be captured after it; a capture goes without.
+int ensure_scratch(llmtie_decode_scratch* s, size_t part_floats, size_t ctrs, hipStream_t st, size_t room = 0) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return driver("hipGetDevice", e);
     const bool swap = s->device != dev;
-    const bool grow = swap || s->part_cap < part_floats || s->ctr_cap < ctrs;
-    if (!grow) return LLMTIE_OK;
+    const bool fits = !swap && s->part_cap >= part_floats && s->ctr_cap >= ctrs;
+    if (fits && s->part_cap >= room) return LLMTIE_OK;
     // Allocating inside a stream capture would put the allocation into the
     // graph (or fail); the caller makes one eager call first instead.
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     e = hipStreamIsCapturing(st, &cs);
     if (e != hipSuccess) return driver("hipStreamIsCapturing", e);
+    if (cs != hipStreamCaptureStatusNone && fits) return LLMTIE_OK;
     if (cs != hipStreamCaptureStatusNone)
         return fail(LLMTIE_SCRATCH_GROWTH_IN_CAPTURE, part_floats, s->part_cap, ctrs, s->ctr_cap,
                     "the decode scratch must grow to %zu partial floats and %zu counters while the stream is "
                     "capturing a graph; make one call of this shape before capturing",
                     part_floats, ctrs);
+    part_floats = std::max(part_floats, room);
     int r;
     if (swap) {
         // A scratch follows the device it is used on; switching starts over.
@@ -550,7 +554,15 @@ int decode_common(void* stream, int kind, const float* q, size_t q_len, size_t q
         part_p = f.part;
         ctr_p = f.ctr;
     } else {
-        int r = ensure_scratch(scratch, part, kv_heads * CTR_STRIDE, S(stream));
+        // A context that the rule keeps whole makes room for the splits it
+        // would take past twelve blocks, as its neighbours past the line do.
+        size_t room = 0;
+        if (one && (tk + 31) / 32 > 12) {
+            int nit2, splits2;
+            plan_decode(tk, kv_heads, group, nit2, splits2);
+            room = kv_heads * ((size_t)splits2 * group * hd + ml_stride(splits2, group));
+        }
+        int r = ensure_scratch(scratch, part, kv_heads * CTR_STRIDE, S(stream), room);
         if (r != LLMTIE_OK) return r;
         part_p = scratch->part;
         ctr_p = scratch->ctr;
