@@ -222,3 +222,38 @@ def test_a_prefill_without_memory_for_its_workspace_is_not_split(monkeypatch):
 
     monkeypatch.setattr(torch, "empty", full)
     assert g._flash_ws(173, 3011, 32, 8, 128) is None
+
+
+@pytest.mark.parametrize("tiled", [False, True])
+def test_a_prefill_with_memory_for_its_output_alone_is_answered(monkeypatch, tiled):
+    """The workspace takes no memory that the output needs."""
+    import types
+    import torch
+    import ttsxabe_amd.gpu as G
+    tq, past, heads, kv, hd, cap = 173, 3011, 32, 8, 128, 4096
+    out = tq * heads * hd
+    # Either of the two fits, not both.
+    room = [_lib.lib().llmtie_flash_attn_workspace(tq, past, heads, kv, hd) + out // 2]
+    calls, empty = [], torch.empty
+
+    def limited(n, **k):
+        if n > room[0]:
+            raise torch.OutOfMemoryError("out of memory")
+        room[0] -= n
+        return empty(n, **k)
+
+    ok = lambda *a: calls.append(a) or 0
+    g = G.Gpu.__new__(G.Gpu)
+    g.device = torch.device("cpu")
+    g._L = types.SimpleNamespace(llmtie_flash_attn_workspace=_lib.lib().llmtie_flash_attn_workspace,
+                                 llmtie_flash_attn_f16_ws=ok, llmtie_flash_attn_t16_ws=ok)
+    monkeypatch.setattr(G, "_need", lambda *a: None)
+    monkeypatch.setattr(G.Gpu, "_stream", lambda self: 0)
+    monkeypatch.setattr(torch, "empty", limited)
+    one = torch.zeros(1)
+    if tiled:
+        cache = types.SimpleNamespace(data=one, kv_heads=kv, head_dim=hd, cap=cap)
+        got = g.flash_attn_t16(one, cache, tq, past, heads, 0.088, True)
+    else:
+        got = g.flash_attn_f16(one, one, one, tq, past, heads, kv, hd, cap, 0.088, True)
+    assert got.numel() == out and len(calls) == 1 and calls[0][-2:] == (None, 0)

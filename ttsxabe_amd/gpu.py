@@ -238,11 +238,15 @@ class Gpu:
     def supports_flash(self, head_dim: int, heads: int, kv_heads: int) -> bool:
         return bool(self._L.llmtie_supports_flash(head_dim, heads, kv_heads))
 
-    def _flash(self, fn, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale, causal, kdt, *ws):
+    def _flash(self, fn, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale, causal, kdt, *ws, split=False):
         _need(q, _F32, "q")
         _need(k, kdt, "k")
         _need(v, kdt, "v")
         out = torch.empty(max(tq * heads * head_dim, 1), dtype=torch.float32, device=self.device)
+        # After the output: a card with room for that alone still has its call.
+        if split:
+            w = self._flash_ws(tq, past, heads, kv_heads, head_dim)
+            ws = _p(w), _n(w)
         _check(fn(self._stream(), _p(q), _n(q), _p(k), _n(k), _p(v), _n(v), _p(out), tq * heads * head_dim, tq, past,
                   heads, kv_heads, head_dim, cap, scale, int(bool(causal)), *ws))
         return out[: tq * heads * head_dim]
@@ -269,9 +273,8 @@ class Gpu:
 
     def flash_attn_f16(self, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale, causal):
         """device.rs:5754. k, v: f16 caches (float16 or 16-bit integer bits)."""
-        ws = self._flash_ws(tq, past, heads, kv_heads, head_dim)
         return self._flash(self._L.llmtie_flash_attn_f16_ws, q, k, v, tq, past, heads, kv_heads, head_dim, cap, scale,
-                           causal, _H16, _p(ws), _n(ws))
+                           causal, _H16, split=True)
 
     def flash_attn_rows(self, qkv, t, heads, head_dim, scale):
         """device.rs:5812. Returns the f16 context [t * heads * head_dim]."""
