@@ -133,7 +133,8 @@ int llmtie_flash_attn_f16(void* stream, const float* q, size_t q_len, const uint
  * launches of few rows over many keys (a turn of a long conversation), whose
  * keys are then cut into runs attended by workgroups of their own and merged
  * in a second launch. llmtie_flash_attn_workspace gives the floats such a call
- * needs (0: the shape is not split, and no workspace is needed). The workspace
+ * needs (0: the shape is not split, and no workspace is needed; never more than
+ * 64 * 16 * (head_dim + 2) a compute unit, 136 MB at head_dim 128). The workspace
  * is written and read on `stream` by this call alone and may be reused or
  * freed in stream order after it; concurrent calls need one each. `ws` NULL is
  * the plain call. A workspace shorter than needed is refused as

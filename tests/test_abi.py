@@ -205,8 +205,13 @@ def test_the_prefill_workspace_is_asked_for_where_keys_outnumber_rows():
     for shape in [(16, 3000, 32, 8, 96), (16, 3000, 33, 8, 128), (16, 3000, 32, 0, 128), (16, W - 8, 32, 8, 128),
                   (W - 1, 3000, 32, 8, 128), (16, 3000, 2**60, 2**60, 128)]:
         assert need(*shape) == 0, shape
-    # Never more than about 800 workgroups' 64 rows of partials.
-    assert max(need(t, p, 32, 8, 128) for t in range(1, 700, 13) for p in range(0, 8000, 533)) <= 800 * 64 * 130
+    # Never more than the partials of 16 workgroups of 64 (row, head)s a compute
+    # unit, at any group and up to a few million positions.
+    for heads, kv, hd in [(32, 8, 128), (40, 40, 128), (32, 8, 64), (8, 2, 128), (16, 8, 128), (20, 20, 64),
+                          (64, 4, 128), (71, 71, 128)]:
+        sizes = [need(t, p, heads, kv, hd) for t in range(1, 2200, 37)
+                 for p in (0, 533, 3011, 7979, 30250, 129000, 3000000)]
+        assert 0 < max(sizes) <= 16 * 256 * 64 * (hd + 2), (heads, kv, hd)
 
 
 def test_a_prefill_without_memory_for_its_workspace_is_not_split(monkeypatch):

@@ -183,7 +183,11 @@ int pick_nqt(size_t tq, size_t heads, int gb, bool staged = false) {
 // 13.1 / 19.5. Where the model keeps one run, two or three measured slower: 300
 // rows after 700, 24 / 20; 64 after 448, 11.6 / 11.1; 400 after 1500 of
 // 40/40/128, 49 / 42; 2000 first rows of 8/2/128, 33-35 / 34.
-constexpr size_t PREFILL_MAX_SPLITS = 32;
+// The partials are bounded by the workgroups: 64 (row, head)s each, at most 16 a
+// compute unit, 136 MB at head_dim 128 on 256 units, which only turns past
+// 30000 positions come near (526 rows after 129000 of 32/8/128, 22 runs 1344 us,
+// whole 1887).
+constexpr size_t PREFILL_MAX_SPLITS = 32, PREFILL_MAX_SPLIT_WGS = 16;  // the latter a compute unit
 size_t plan_prefill_splits(size_t tq, size_t past, size_t heads, size_t kv_heads, size_t hd) {
     if (getenv("LLMTIE_PREFILL_NQT")) return 1;
     const size_t group = heads / kv_heads;
@@ -201,6 +205,7 @@ size_t plan_prefill_splits(size_t tq, size_t past, size_t heads, size_t kv_heads
     double least = 0.0;
     for (size_t n = 1; n <= PREFILL_MAX_SPLITS && n <= tiles; ++n) {
         const double load = items * (double)n / cus;
+        if (n > 1 && load > (double)PREFILL_MAX_SPLIT_WGS) break;
         const double period = load <= 1.0 ? 0.95 : load <= 2.0 ? 0.95 + 0.55 * (load - 1.0) : 0.75 * std::ceil(load);
         const double us = (double)((tiles + n - 1) / n) * period * tile_us + (n > 1 ? 4.5 + (double)n * run_us : 0.0);
         if (n == 1 || us < least) {
