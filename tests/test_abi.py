@@ -205,6 +205,10 @@ def test_the_prefill_workspace_is_asked_for_where_keys_outnumber_rows():
     for shape in [(16, 3000, 32, 8, 96), (16, 3000, 33, 8, 128), (16, 3000, 32, 0, 128), (16, W - 8, 32, 8, 128),
                   (W - 1, 3000, 32, 8, 128), (16, 3000, 2**60, 2**60, 128)]:
         assert need(*shape) == 0, shape
+    # Nor those that splitting measured slower on.
+    for shape in [(125, 622, 32, 8, 128), (206, 691, 32, 8, 128), (244, 908, 32, 8, 128), (322, 563, 16, 8, 128),
+                  (142, 811, 40, 40, 128), (524, 296, 8, 2, 128), (300, 700, 32, 8, 128)]:
+        assert need(*shape) == 0, shape
     # Never more than the partials of 16 workgroups of 64 (row, head)s a compute
     # unit, at any group and up to a few million positions.
     for heads, kv, hd in [(32, 8, 128), (40, 40, 128), (32, 8, 64), (8, 2, 128), (16, 8, 128), (20, 20, 64),

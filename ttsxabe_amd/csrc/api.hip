@@ -174,14 +174,19 @@ int pick_nqt(size_t tq, size_t heads, int gb, bool staged = false) {
 
 // Runs the tiles of each position block of a prefill off an f16 cache are cut
 // into (1: not split), one workgroup each: the cheapest under a model of the
-// launch fitted to MI355X, in microseconds at head_dim 128. A workgroup's 64-key
-// tile takes 0.95 alone on its compute unit and 1.5 beside a second one (two
-// fit); a third waits. Splitting adds the merge's launch and the partials'
-// traffic, so few rows over many keys split far and many rows or few keys not
-// at all. Measured, split / not: 173 rows after 3011 positions of 32/8/128, 28 /
-// 47 us; 16 after 3000, 14.6 / 44; 100 after 7000, 28 / 95; 40 after 1000,
-// 13.1 / 19.5. Where the model keeps one run, two or three measured slower: 300
-// rows after 700, 24 / 20; 64 after 448, 11.6 / 11.1; 400 after 1500 of
+// launch in microseconds, fitted on MI355X to 700 causal shapes of nine head
+// counts of 64 and 128 timed at up to eleven run counts each. A workgroup's
+// 64-key tile takes 0.95 alone on its compute unit, and where some units hold
+// two workgroups (two fit) those set the pace, 1.2 up to 1.4; a third waits.
+// Splitting adds the merge's launch and the partials' traffic, so few rows over
+// many keys split far and many rows or few keys not at all. On 400 other shapes
+// that it splits, none is slower than whole (one by 2.9 % without the causal
+// mask), the mean 0.48 of its time. Measured, split / not: 173 rows after
+// 3011 positions of 32/8/128, 28-31 / 45-47 us; 16 after 3000, 14.6 / 44; 100
+// after 7000, 28 / 95; 40 after 1000, 13.1 / 19.5; at head_dim 64, 173 after
+// 3011, 19.4 / 40.7; 40 after 1000, 10.9 / 18; 16 after 3000, 12.2 / 39.4. Where
+// it keeps one run, two or three measured slower: 206 rows after 691, 19.4 /
+// 16.9; 125 after 622, 16.0 / 14.3; 300 after 700, 24 / 20; 400 after 1500 of
 // 40/40/128, 49 / 42; 2000 first rows of 8/2/128, 33-35 / 34.
 // The partials are bounded by the workgroups: 64 (row, head)s each, at most 16 a
 // compute unit, 136 MB at head_dim 128 on 256 units, which only turns past
@@ -198,22 +203,23 @@ size_t plan_prefill_splits(size_t tq, size_t past, size_t heads, size_t kv_heads
     if (items > 2 * cus) return 1;
     const size_t tiles = (past + tq + 63) / 64;
     if (tiles <= 8) return 1;  // no shape measured gains; the Python binding does not ask either
-    const double tile_us = hd == 128 ? 1.0 : 0.7;
     // One run's partials written and read, and its share of the merge's chain.
-    const double run_us = (double)(tq * heads * hd) * 8.0 / 5e6 + 0.1;
+    const double run_us = (double)(tq * heads * hd) * 8.0 / 3.1e6 + 0.1;
     size_t best = 1;
-    double least = 0.0;
+    double least = 0.0, whole = 0.0;
     for (size_t n = 1; n <= PREFILL_MAX_SPLITS && n <= tiles; ++n) {
         const double load = items * (double)n / cus;
         if (n > 1 && load > (double)PREFILL_MAX_SPLIT_WGS) break;
-        const double period = load <= 1.0 ? 0.95 : load <= 2.0 ? 0.95 + 0.55 * (load - 1.0) : 0.75 * std::ceil(load);
-        const double us = (double)((tiles + n - 1) / n) * period * tile_us + (n > 1 ? 4.5 + (double)n * run_us : 0.0);
-        if (n == 1 || us < least) {
+        const double period = load <= 1.0 ? 0.95 : load <= 2.0 ? 1.2 + 0.2 * (load - 1.0) : 0.75 * std::ceil(load);
+        const double us = (double)((tiles + n - 1) / n) * period + (n > 1 ? 4.5 + (double)n * run_us : 0.0);
+        if (n == 1) whole = least = us;
+        if (us < least) {
             best = n;
             least = us;
         }
     }
-    return best;
+    // Within 2 % of the whole one the two measured either way.
+    return least < 0.98 * whole ? best : 1;
 }
 
 int prefill_common(void* stream, int kind, const float* q, size_t q_len, const void* k, size_t k_len, const void* v,
