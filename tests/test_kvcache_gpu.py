@@ -337,6 +337,24 @@ def test_rope_of_many_rows_is_each_row_alone_and_nothing_else_moves(gpu, t, head
         assert np.array_equal(down(row)[1:], got[off + p * heads * hd: off + (p + 1) * heads * hd])
 
 
+# Counts at the top of an int, and rows of one head whose workgroups would pass
+# a launch's 2^32 threads: 17 GB each, checked at both ends and around every
+# half that a launch may be cut at.
+@pytest.mark.parametrize("t,heads,hd", [(2**31 - 1, 1, 2), (2**24 + 1, 1, 258), (1, 2**31 - 1, 2)])
+def test_rope_of_the_largest_counts(gpu, t, heads, hd):
+    x = torch.empty(t * heads * hd, device="cuda").uniform_(-1.0, 1.0)
+    units = max(t, heads)
+    at = sorted({min(max(i * units // 16 + d, 0), units - 1) for i in range(17) for d in (-1, 0, 1)})
+    want = {u: x[u * hd:(u + 1) * hd].clone() for u in at}
+    for u in at:
+        gpu.rope(want[u], 0, 1, 1, hd, 10000.0, (u if t > 1 else 7))
+    gpu.rope(x, 0, t, heads, hd, 10000.0, 0 if t > 1 else 7)
+    bad = [u for u in at if not torch.equal(x[u * hd:(u + 1) * hd], want[u])]
+    del x
+    torch.cuda.empty_cache()
+    assert not bad
+
+
 # Position tiles cut on both sides, whole and single ones; capacities whose
 # rows are whole float4s / half4s and not; a source on and off 16 bytes.
 @pytest.mark.parametrize("n,past,cap", [(1, 0, 4), (15, 3, 18), (16, 0, 16), (63, 1, 64), (64, 64, 130), (65, 62, 140),

@@ -639,6 +639,19 @@ hipError_t launch_rope(float* x, long off, const float* div, int t, int heads, i
                        hipStream_t st) {
     const int half = hd / 2;
     if ((long)t * heads * half == 0) return hipSuccess;
+    // The kernel counts in ints and a launch holds fewer than 2^32 threads:
+    // rows of more than 2^23 workgroups, or heads past 2^30, go in halves.
+    const bool many = heads > 1 << 30;
+    if (t > 1 && (many || (long)t * ((half + KB - 1) / KB) > 1L << 23)) {
+        const int lo = t / 2;
+        if (hipError_t e = launch_rope(x, off, div, lo, heads, hd, theta, first, st)) return e;
+        return launch_rope(x, off + (long)lo * heads * hd, div, t - lo, heads, hd, theta, first + lo, st);
+    }
+    if (many) {
+        const int lo = heads / 2;
+        if (hipError_t e = launch_rope(x, off, div, t, lo, hd, theta, first, st)) return e;
+        return launch_rope(x, off + (long)lo * hd, div, t, heads - lo, hd, theta, first, st);
+    }
     // float4 halves where every head's two halves start on one.
     const int vec = half % 4 == 0 && aligned16(x + off) ? 4 : 1;
     // One angle a thread: jn pairs (whole vectors) of pn positions.
