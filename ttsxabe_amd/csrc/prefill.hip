@@ -549,9 +549,9 @@ __device__ __forceinline__ void store_ctx16(float* R, const floatx4 (&o)[WD / 16
 // launches what the first gained. Where the tile reaches past the keys:
 //   PF_T16: both its halves come from its first block when that is the last
 //     one a row sees, so every address lies in a live block;
-//   PF_F16: K rows up to the capacity are read as they lie and rows past it,
-//     like V past the allocation, are out of the resource's range (every
-//     offset is in the lane's, which the range check covers): zeros.
+//   PF_F16: K rows past the keys, like V past the allocation, are out of the
+//     resource's range (every offset is in the lane's, which the range check
+//     covers): zeros, whatever lies there.
 // Those scores are masked and V past ktot is zeroed in LDS.
 // 32/8/128 causal, before -> this: tiled cache, 8192 / 1999 / 512 / 128 rows
 // 539 -> 525, 54.2 -> 50.5, 13.2 -> 12.4, 6.7 -> 6.2 us; reference layout, 8192
@@ -567,7 +567,7 @@ struct TileLoad {
 
     const half_t* kc;
     size_t hb;           // PF_T16: the head's first block; PF_F16: the kv head
-    int cap;
+    int cap, ktot;
     const char* v;
     uint32_t v_bytes;
     int w0;              // the wave, as a scalar
@@ -578,6 +578,7 @@ struct TileLoad {
         : kc(static_cast<const half_t*>(a.k)),
           hb(KIND == PF_T16 ? (size_t)kh * tiled_nblk(a.cap) : (size_t)kh),
           cap(a.cap),
+          ktot(a.past + a.tq),
           v(static_cast<const char*>(a.v)),
           v_bytes((uint32_t)a.v_bytes),
           w0(__builtin_amdgcn_readfirstlane(wave)),
@@ -616,7 +617,7 @@ struct TileLoad {
         } else {
             const size_t vb = (hb * HD * cap + kv0) * 2;
             const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<half_t*>(kc) + (hb * cap + kv0) * HD, 0, min(cap - kv0, KT) * (2 * HD), 0x00020000);
+                const_cast<half_t*>(kc) + (hb * cap + kv0) * HD, 0, min(ktot - kv0, KT) * (2 * HD), 0x00020000);
             const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
                 const_cast<char*>(v) + vb, 0, (int)(v_bytes - (uint32_t)vb), 0x00020000);
 #pragma unroll
