@@ -205,7 +205,9 @@ def test_the_prefill_workspace_is_asked_for_where_keys_outnumber_rows():
     for shape in [(16, 3000, 32, 8, 96), (16, 3000, 33, 8, 128), (16, 3000, 32, 0, 128), (16, W - 8, 32, 8, 128),
                   (W - 1, 3000, 32, 8, 128), (16, 3000, 2**60, 2**60, 128)]:
         assert need(*shape) == 0, shape
-    # Nor those that splitting measured slower on.
+    # Many rows whose halves still fit the chip do.
+    assert need(353, 2019, 32, 8, 128) == 2 * 353 * 32 * 130 and need(325, 3180, 40, 40, 128)
+    # Not those that splitting measured slower on.
     for shape in [(125, 622, 32, 8, 128), (206, 691, 32, 8, 128), (244, 908, 32, 8, 128), (322, 563, 16, 8, 128),
                   (142, 811, 40, 40, 128), (524, 296, 8, 2, 128), (300, 700, 32, 8, 128)]:
         assert need(*shape) == 0, shape

@@ -174,14 +174,17 @@ int pick_nqt(size_t tq, size_t heads, int gb, bool staged = false) {
 
 // Runs the tiles of each position block of a prefill off an f16 cache are cut
 // into (1: not split), one workgroup each: the cheapest under a model of the
-// launch in microseconds, fitted on MI355X to 700 causal shapes of nine head
-// counts of 64 and 128 timed at up to eleven run counts each. A workgroup's
-// 64-key tile takes 0.95 alone on its compute unit, and where some units hold
-// two workgroups (two fit) those set the pace, 1.2 up to 1.4; a third waits.
+// launch in microseconds, fitted on MI355X to 2700 causal shapes of nine head
+// counts of 64 and 128, half of them timed at up to eleven run counts. A
+// workgroup's 64-key tile takes 0.86 on an empty chip and 0.24 more for each
+// workgroup a compute unit holds, up to two; further ones wait. Counts that do
+// not deal whole eighths to the XCDs' L2s cost 13 % a tile; a whole launch of
+// head_dim 64 that fills half the units saves 10 %.
 // Splitting adds the merge's launch and the partials' traffic, so few rows over
-// many keys split far and many rows or few keys not at all. On 400 other shapes
-// that it splits, none is slower than whole (one by 2.9 % without the causal
-// mask), the mean 0.48 of its time. Measured, split / not: 173 rows after
+// many keys split far and many rows or few keys not at all. Four of those
+// shapes are slower than whole by more than 1 %, the worst 6.2 % (17 rows after
+// 513 of 40/40/128, 13.55 / 12.76); of 500 others two, 1.8 %, the mean 0.47 of
+// the whole one's time. Measured, split / not: 173 rows after
 // 3011 positions of 32/8/128, 28-31 / 45-47 us; 16 after 3000, 14.6 / 44; 100
 // after 7000, 28 / 95; 40 after 1000, 13.1 / 19.5; at head_dim 64, 173 after
 // 3011, 19.4 / 40.7; 40 after 1000, 10.9 / 18; 16 after 3000, 12.2 / 39.4. Where
@@ -204,22 +207,25 @@ size_t plan_prefill_splits(size_t tq, size_t past, size_t heads, size_t kv_heads
     const size_t tiles = (past + tq + 63) / 64;
     if (tiles <= 8) return 1;  // no shape measured gains; the Python binding does not ask either
     // One run's partials written and read, and its share of the merge's chain.
-    const double run_us = (double)(tq * heads * hd) * 8.0 / 3.1e6 + 0.1;
+    const double run_us = (double)(tq * heads * hd) * 8.0 / 3.1e6 + 0.11;
     size_t best = 1;
     double least = 0.0, whole = 0.0;
     for (size_t n = 1; n <= PREFILL_MAX_SPLITS && n <= tiles; ++n) {
         const double load = items * (double)n / cus;
         if (n > 1 && load > (double)PREFILL_MAX_SPLIT_WGS) break;
-        const double period = load <= 1.0 ? 0.95 : load <= 2.0 ? 1.2 + 0.2 * (load - 1.0) : 0.75 * std::ceil(load);
-        const double us = (double)((tiles + n - 1) / n) * period + (n > 1 ? 4.5 + (double)n * run_us : 0.0);
+        double period = load <= 2.0 ? 0.86 + 0.24 * load : 0.67 * std::ceil(load);
+        if ((size_t)items * n % 8 != 0) period *= 1.13;
+        if (n == 1 && hd == 64 && 2 * items > cus) period *= 0.9;
+        const double merge_us = n == 1 ? 0.0 : (load <= 1.0 ? 3.4 : 5.4) + (double)n * run_us;
+        const double us = (double)((tiles + n - 1) / n) * period + merge_us;
         if (n == 1) whole = least = us;
         if (us < least) {
             best = n;
             least = us;
         }
     }
-    // Within 2 % of the whole one the two measured either way.
-    return least < 0.98 * whole ? best : 1;
+    // Within 5 % of the whole one the two measured either way.
+    return least < 0.95 * whole ? best : 1;
 }
 
 int prefill_common(void* stream, int kind, const float* q, size_t q_len, const void* k, size_t k_len, const void* v,
