@@ -73,3 +73,55 @@ def test_a_head_spread_over_xcds_is_nan_and_reported(gpu):
     with pytest.raises(SplitHeadLost):
         s.check()
     s.check()  # cleared
+
+
+def _q8(gpu, nseq, kv, s, monkeypatch, static=None):
+    from tests.test_q8_decode_gpu import load, random_q8_cache
+    from ttsxabe_amd.gpu import KvCacheQ8
+    heads, hd, cap = 4 * kv, 128, 2048
+    if static is not None:
+        monkeypatch.setenv("LLMTIE_DECODE_STATIC", static)
+    cache = KvCacheQ8(nseq, kv, hd, cap)
+    load(cache, *random_q8_cache(nseq, kv, hd, cap, 51))
+    q = up(oracle.normal(nseq * heads * hd, 52))
+    tk = up(oracle.uniform_int(nseq, 53, 1100, 2000).astype(np.int32), torch.int32)
+    slot = up(np.arange(nseq, dtype=np.int32), torch.int32)
+    return lambda: down(gpu.attn_decode_q8_batch(q, cache, tk, slot, 2000, heads, 0.088, False, s))
+
+
+@pytest.mark.parametrize("static", [None, "0", "1"])
+@pytest.mark.parametrize("nseq,kv", [(8, 8), (32, 2)])
+def test_no_head_of_a_batch_of_64_sequences_depends_on_an_xcd(gpu, nseq, kv, static, monkeypatch):
+    from ttsxabe_amd import _lib
+    from ttsxabe_amd.gpu import DecodeScratch
+    s = DecodeScratch()
+    run = _q8(gpu, nseq, kv, s, monkeypatch, static)
+    good = run()
+    assert np.isfinite(good).all()
+    _lib.lib().llmtie_debug_fake_xcc(1)
+    try:
+        again = run()
+    finally:
+        _lib.lib().llmtie_debug_fake_xcc(0)
+    assert np.array_equal(good.view(np.uint32), again.view(np.uint32))
+    s.check()
+
+
+def test_a_larger_batch_hands_over_in_one_xcd_and_says_when_it_could_not(gpu, monkeypatch):
+    from ttsxabe_amd import _lib
+    from ttsxabe_amd.gpu import DecodeScratch, SplitHeadLost
+    s = DecodeScratch()
+    run = _q8(gpu, 72, 2, s, monkeypatch)  # 144 heads in three splits: whole heads an XCD
+    local = run()
+    _lib.lib().llmtie_debug_fake_xcc(1)
+    try:
+        bad = run()
+    finally:
+        _lib.lib().llmtie_debug_fake_xcc(0)
+    assert np.isnan(bad).all(), "every head is merged across splits"
+    with pytest.raises(SplitHeadLost):
+        run()
+    monkeypatch.setenv("LLMTIE_DECODE_XCD", "0")
+    coherent = run()
+    assert np.isfinite(local).all()
+    assert np.array_equal(local.view(np.uint32), coherent.view(np.uint32))
