@@ -51,7 +51,8 @@ typedef enum llmtie_status {
     LLMTIE_ODD_HEAD_DIM = 7,          /* OddHeadDim{head_dim}             error.rs:210 */
     LLMTIE_DRIVER = 8,                /* Driver{what, source}             error.rs:281 */
     LLMTIE_NO_DEVICE = 9,             /* NoDevice(String)                 error.rs:242 */
-    LLMTIE_INVALID_ARGUMENT = 10,     /* a null pointer where a buffer is required (no reference twin) */
+    LLMTIE_INVALID_ARGUMENT = 10,     /* a null pointer where a buffer is required, or a prefill
+                                        * workspace off 16 bytes (no reference twin) */
     LLMTIE_SCRATCH_GROWTH_IN_CAPTURE = 11, /* a decode scratch would have to grow while its stream captures a
                                             * graph (no reference twin: the reference does not capture);
                                             * fields: partial floats needed, held, counters needed, held */
@@ -138,7 +139,8 @@ int llmtie_flash_attn_f16(void* stream, const float* q, size_t q_len, const uint
  * is written and read on `stream` by this call alone and may be reused or
  * freed in stream order after it; concurrent calls need one each. `ws` NULL is
  * the plain call. A workspace shorter than needed is refused as
- * LLMTIE_SLICE_OVERRUN. It is 16-byte aligned. */
+ * LLMTIE_SLICE_OVERRUN, one that is not 16-byte aligned as
+ * LLMTIE_INVALID_ARGUMENT. */
 size_t llmtie_flash_attn_workspace(size_t tq, size_t past, size_t heads, size_t kv_heads, size_t head_dim);
 int llmtie_flash_attn_f16_ws(void* stream, const float* q, size_t q_len, const uint16_t* k, size_t k_len,
                              const uint16_t* v, size_t v_len, float* out, size_t out_len, size_t tq, size_t past,

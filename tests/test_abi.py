@@ -220,6 +220,17 @@ def test_the_prefill_workspace_is_asked_for_where_keys_outnumber_rows():
         assert 0 < max(sizes) <= 16 * 256 * 64 * (hd + 2), (heads, kv, hd)
 
 
+def test_a_workspace_off_16_bytes_is_refused():
+    L = _lib.lib()
+    P, big = 4096, 10**9
+    for off in (4, 8, 12):
+        assert L.llmtie_flash_attn_f16_ws(NULL, P, big, P, big, P, big, P, big, 16, 3000, 32, 8, 128, 4096, 0.1, 1,
+                                          P + off, big) == 10
+        assert b"16 bytes" in last().message
+        assert L.llmtie_flash_attn_t16_ws(NULL, P, big, P, big, P, big, 16, 3000, 32, 8, 128, 4096, 0.1, 1, P + off,
+                                          big) == 10
+
+
 def test_a_prefill_without_memory_for_its_workspace_is_not_split(monkeypatch):
     """A full card refuses the workspace, not the call."""
     import torch

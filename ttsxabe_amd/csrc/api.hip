@@ -268,6 +268,8 @@ int prefill_common(void* stream, int kind, const float* q, size_t q_len, const v
     if (splits > 1) {
         const size_t need = smul(smul(splits, tq, heads), hd + 2);
         if (ws_len < need) return overrun_slice(need, ws_len);
+        if (reinterpret_cast<uintptr_t>(ws) % 16 != 0)
+            return fail(LLMTIE_INVALID_ARGUMENT, 0, 0, 0, 0, "a workspace off 16 bytes");
         a.splits = (int)splits;
         a.ws = ws;
         nqt = 1;
