@@ -171,3 +171,28 @@ def test_stream_k_and_the_planned_grid_are_the_same_attention(gpu, hd, heads, kv
     n = len(lengths)
     check_batch(gpu, hd, heads, kv, n, 2528, np.array(lengths, np.int32), np.arange(n, dtype=np.int32)[::-1].copy(),
                 45 + n)
+
+
+# What the planned grid measured slower on than stream-K (several rounds of
+# split heads), beside shapes of one round, of fewer bytes and of whole heads
+# that it is faster on: stream-K's bits are its own.
+@pytest.mark.parametrize("hd,heads,kv,nseq,high,stream_k", [
+    (128, 32, 8, 17, 1646, True), (128, 16, 8, 25, 1050, True), (128, 40, 40, 4, 1281, True),
+    (128, 40, 40, 3, 2276, True), (128, 32, 8, 14, 1681, False), (128, 16, 8, 19, 1060, False),
+    (64, 32, 8, 17, 1129, False), (128, 16, 8, 54, 471, False)])
+def test_batches_run_on_the_grid_that_is_faster(gpu, hd, heads, kv, nseq, high, stream_k, monkeypatch):
+    from ttsxabe_amd.gpu import DecodeScratch, KvCacheQ8
+    cache = KvCacheQ8(nseq, kv, hd, high)
+    blocks = cache.data.view(-1, 68 * hd)
+    blocks[:, :64 * hd].random_(-128, 127)
+    blocks[:, 64 * hd:] = torch.full((blocks.shape[0], 2 * hd), 0.01, dtype=torch.float16,
+                                     device="cuda").view(torch.int8)
+    q = up(oracle.normal(nseq * heads * hd, 61))
+    tk = up(np.linspace(high // 2, high, nseq).astype(np.int32), torch.int32)
+    slot = up(np.arange(nseq, dtype=np.int32), torch.int32)
+    run = lambda: down(gpu.attn_decode_q8_batch(q, cache, tk, slot, high, heads, hd ** -0.5, False, DecodeScratch()))
+    got = run()
+    monkeypatch.setenv("LLMTIE_DECODE_STATIC", "0")
+    sk = run()
+    assert np.array_equal(got, sk) == stream_k
+    assert full_scale_err(sk, got) < 2e-3  # each within 1e-3 of the exact value

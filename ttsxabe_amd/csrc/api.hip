@@ -375,15 +375,21 @@ bool plan_q8_batch(size_t nseq, size_t kv_heads, size_t hd, size_t max_tk, int& 
     const size_t units = nseq * kv_heads;
     const double mb = (double)units * (double)max_tk * (double)(2 * hd + hd / 8) * 1e-6;
     if (mb > (units <= 64 ? 150.0 : 75.0)) return true;
-    // Beyond one round of workgroups, spans of 1024 keys (eight blocks a wave):
-    // 12 sequences of 100-1000, 10.8 us against 14.0 in three splits each; 20,
-    // 12.6 / 15.5; 32, 14.2 / 20.9.
+    // Beyond one round of workgroups, even spans of up to 1024 keys (eight blocks
+    // a wave): 12 sequences of 100-1000, 10.8 us against 14.0 in three splits
+    // each; 20, 12.6 / 15.5; 32, 14.2 / 20.9.
     if (units > 64 && units * (size_t)splits > 256 && nit < 8 && !getenv("LLMTIE_DECODE_NIT") &&
         !getenv("LLMTIE_DECODE_WGS")) {
-        nit = 8;
-        splits = (int)((max_tk + 1023) / 1024);
+        const size_t spans = (max_tk + 1023) / 1024;
+        nit = (int)(((max_tk + 31) / 32 + 4 * spans - 1) / (4 * spans));
+        splits = (int)((max_tk + 128 * (size_t)nit - 1) / (128 * (size_t)nit));
     }
-    return false;
+    // Several such rounds of split heads at head_dim 128 lose to stream-K from
+    // 45 MB on: 17 sequences of up to 1646 over 8 kv heads, 23.8 / 20.5 us; 25 of
+    // 1050, 21.4 / 18.9; 19 of 1174 (48 MB), 19.2 / 17.8; 4 of 1281 over 40, 20.4 /
+    // 18.9; but 14 of 1681 over 8 (one round), 17.8 / 21.0; 19 of 1088 (45 MB),
+    // 15.6 / 16.8.
+    return hd == 128 && splits > 1 && units * (size_t)splits > 256 && mb > 45.0;
 }
 
 // Whether the split partials are merged by a second launch rather than by
