@@ -16,7 +16,7 @@ import pytest
 import torch
 
 import oracle
-from tests.test_q8_decode_gpu import dequant_seq, load, random_q8_cache
+from tests.test_q8_decode_gpu import both_grids, dequant_seq, grid, load, random_q8_cache
 from tests.util import down, full_scale_err, up, up_f16
 
 pytestmark = pytest.mark.gpu
@@ -39,9 +39,11 @@ def test_wide_groups_and_short_contexts(gpu, heads, kv, hd, tk, cap):
     assert np.array_equal(a, down(gpu.attn_decode_t16(up(q), t, heads, tk, 0.09, False, s)))
 
 
+@both_grids
 @pytest.mark.parametrize("nseq", [1, 64, 65])
-def test_q8_batch_at_the_edges_of_its_plan(gpu, nseq):
+def test_q8_batch_at_the_edges_of_its_plan(gpu, nseq, static, monkeypatch):
     from ttsxabe_amd.gpu import DecodeScratch, KvCacheQ8
+    grid(monkeypatch, static)
     hd, heads, kv, slots, cap = 128, 8, 2, 7, 512
     kc, ks, vc, vs = random_q8_cache(slots, kv, hd, cap, 61)
     cache = KvCacheQ8(slots, kv, hd, cap)

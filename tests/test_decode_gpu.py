@@ -283,3 +283,21 @@ def test_one_call_has_one_result_whatever_room_its_scratch_has(gpu, heads, kv, t
         assert torch.equal(got, want)
     exact = oracle.decode_f64(q, oracle.through_f16(k), oracle.through_f16(v), heads, kv, hd, tk, cap, scale, False)
     assert np.abs(exact - down(want)).max() / np.abs(exact).max() < 2e-5
+
+
+def test_the_two_layouts_are_bit_equal_where_they_take_one_plan(gpu):
+    """At head_dim 128 the reference layout splits contexts of ten to twelve
+    blocks that the tiled one keeps whole: there the sums have another order."""
+    from ttsxabe_amd.gpu import DecodeScratch, TiledCache16
+    heads, kv, hd, cap, s = 8, 2, 128, 448, DecodeScratch()
+    q, k, v = (oracle.seq(n, 71 + i) for i, n in enumerate((heads * hd, kv * cap * hd, kv * cap * hd)))
+    dq, dk, dv = up(q), up_f16(k), up_f16(v)
+    t = TiledCache16(kv, hd, cap)
+    for tk in (1, 128, 129, 288, 289, 384, 385, 448):
+        gpu.t16_from_ref(dk, dv, t, tk)
+        a = down(gpu.attn_decode_f16(dq, dk, dv, heads, kv, hd, tk, cap, 0.088, False, s))
+        b = down(gpu.attn_decode_t16(dq, t, heads, tk, 0.088, False, s))
+        assert np.array_equal(a, b) or 288 < tk < 385, tk
+        exact = oracle.decode_f64(q, oracle.through_f16(k), oracle.through_f16(v), heads, kv, hd, tk, cap, 0.088,
+                                  False)
+        assert full_scale_err(exact, a) < 2e-5 and full_scale_err(exact, b) < 2e-5, tk

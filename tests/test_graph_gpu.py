@@ -66,12 +66,14 @@ def test_prefill_graph_replays(gpu):
                             gpu.flash_attn(q, k32, v32, tq, 0, heads, kv, hd, cap, 0.088, True)])
 
 
-def test_batched_q8_decode_graph_replays(gpu):
-    """The stream-K decode: its mergers leave the arrival counters at zero
-    in the kernel, so every replay starts clean (scratch grown by the eager
-    call first)."""
+@pytest.mark.parametrize("static", [None, "0"])
+def test_batched_q8_decode_graph_replays(gpu, static, monkeypatch):
+    """On the planned grid and on stream-K: the mergers leave the arrival
+    counters at zero in the kernel, so every replay starts clean (scratch grown
+    by the eager call first)."""
     from ttsxabe_amd.gpu import DecodeScratch, KvCacheQ8
-    from tests.test_q8_decode_gpu import load, random_q8_cache
+    from tests.test_q8_decode_gpu import grid, load, random_q8_cache
+    grid(monkeypatch, static)
     hd, heads, kv, slots, cap = 128, 32, 8, 6, 1024
     cache = KvCacheQ8(slots, kv, hd, cap)
     load(cache, *random_q8_cache(slots, kv, hd, cap, 31))

@@ -16,6 +16,16 @@ from tests.util import down, full_scale_err, up
 pytestmark = pytest.mark.gpu
 
 
+# A batch of up to 64 sequences runs on the host-planned grid or stream-K by the
+# bytes its length bound allows: the default rule, and stream-K forced.
+both_grids = pytest.mark.parametrize("static", [None, "0"])
+
+
+def grid(monkeypatch, static):
+    if static is not None:
+        monkeypatch.setenv("LLMTIE_DECODE_STATIC", static)
+
+
 def random_q8_cache(slots, kv, hd, cap, seed):
     n = slots * kv * cap * hd
     kc = (oracle.uniform_int(n, seed, -127, 127)).astype(np.int8)
@@ -42,9 +52,12 @@ def dequant_seq(kc, ks, vc, vs, slot, kv, hd, cap):
     return np.ascontiguousarray(k, np.float32).ravel(), np.ascontiguousarray(v, np.float32).ravel()
 
 
+@both_grids
 @pytest.mark.parametrize("hd,heads,kv,scale_q", [(128, 32, 8, False), (64, 20, 20, True), (128, 8, 8, False)])
-def test_batched_q8_decode_matches_the_chain_on_the_dequantised_cache(gpu, hd, heads, kv, scale_q):
+def test_batched_q8_decode_matches_the_chain_on_the_dequantised_cache(gpu, hd, heads, kv, scale_q, static,
+                                                                      monkeypatch):
     from ttsxabe_amd.gpu import DecodeScratch, KvCacheQ8
+    grid(monkeypatch, static)
     slots, cap, nseq = 6, 1024, 5
     kc, ks, vc, vs = random_q8_cache(slots, kv, hd, cap, 900 + hd)
     cache = KvCacheQ8(slots, kv, hd, cap)
@@ -73,8 +86,10 @@ def test_batched_q8_decode_matches_the_chain_on_the_dequantised_cache(gpu, hd, h
         assert full_scale_err(chain, g) < 1e-3 + own, f"seq {i}"
 
 
-def test_a_mis_described_sequence_gets_nan_and_its_neighbours_do_not(gpu):
+@both_grids
+def test_a_mis_described_sequence_gets_nan_and_its_neighbours_do_not(gpu, static, monkeypatch):
     from ttsxabe_amd.gpu import DecodeScratch, KvCacheQ8
+    grid(monkeypatch, static)
     hd, heads, kv, slots, cap = 128, 8, 2, 2, 64
     cache = KvCacheQ8(slots, kv, hd, cap)
     load(cache, *random_q8_cache(slots, kv, hd, cap, 5))
@@ -127,20 +142,26 @@ def check_batch(gpu, hd, heads, kv, slots, cap, tk, slot, seed, scale_q=False):
         assert full_scale_err(exact, got[i * n:(i + 1) * n]) < 1e-3, f"seq {i} (tk {tk[i]})"
 
 
-def test_many_one_block_heads(gpu):
-    """64 sequences of 1..40 keys: every wave's range holds many whole heads
-    and segments that begin while another segment's queries are pending."""
+@both_grids
+def test_many_one_block_heads(gpu, static, monkeypatch):
+    """64 sequences of 1..40 keys: every stream-K wave's range holds many whole
+    heads and segments that begin while another segment's queries are pending."""
+    grid(monkeypatch, static)
     tk = (oracle.uniform_int(64, 31, 1, 40)).astype(np.int32)
     check_batch(gpu, 128, 32, 8, 64, 64, tk, np.arange(64, dtype=np.int32)[::-1].copy(), 40)
 
 
-def test_one_long_sequence_many_contributors(gpu):
-    """One sequence of 8191 keys: every head is shared by more waves than one
-    merge batch holds."""
+@both_grids
+def test_one_long_sequence_many_contributors(gpu, static, monkeypatch):
+    """One sequence of 8191 keys: under stream-K every head is shared by more
+    waves than one merge batch holds."""
+    grid(monkeypatch, static)
     check_batch(gpu, 128, 32, 8, 1, 8192, np.array([8191], np.int32), np.array([0], np.int32), 41)
 
 
-def test_ragged_mix_and_head_width_64(gpu):
+@both_grids
+def test_ragged_mix_and_head_width_64(gpu, static, monkeypatch):
+    grid(monkeypatch, static)
     tk = (oracle.uniform_int(33, 32, 1, 3000)).astype(np.int32)
     check_batch(gpu, 64, 16, 4, 33, 3008, tk, np.arange(33, dtype=np.int32), 42, scale_q=True)
 
@@ -150,9 +171,11 @@ def test_more_than_64_sequences_take_the_planned_grid(gpu):
     check_batch(gpu, 128, 8, 2, 70, 320, tk, np.arange(70, dtype=np.int32), 43)
 
 
+@both_grids
 @pytest.mark.parametrize("hd,heads,kv", [(128, 16, 1), (64, 8, 8), (128, 64, 4)])
-def test_group_widths(gpu, hd, heads, kv):
-    """GQA groups of 16 (the largest query buffers) and 1 (MHA)."""
+def test_group_widths(gpu, hd, heads, kv, static, monkeypatch):
+    """GQA groups of 16 (stream-K's largest query buffers) and 1 (MHA)."""
+    grid(monkeypatch, static)
     tk = (oracle.uniform_int(9, 34 + heads, 1, 700)).astype(np.int32)
     check_batch(gpu, hd, heads, kv, 9, 704, tk, np.arange(9, dtype=np.int32)[::-1].copy(), 44 + heads)
 
@@ -166,8 +189,7 @@ def test_group_widths(gpu, hd, heads, kv):
     (128, 32, 8, [2500]), (128, 8, 8, [1, 32, 33, 700, 64]), (64, 16, 4, [1, 31, 900, 320, 257]),
     (128, 16, 8, [1, 1023, 1024, 1025, 129, 40, 1500, 600, 31, 32, 33, 777])])
 def test_stream_k_and_the_planned_grid_are_the_same_attention(gpu, hd, heads, kv, lengths, static, monkeypatch):
-    if static is not None:
-        monkeypatch.setenv("LLMTIE_DECODE_STATIC", static)
+    grid(monkeypatch, static)
     n = len(lengths)
     check_batch(gpu, hd, heads, kv, n, 2528, np.array(lengths, np.int32), np.arange(n, dtype=np.int32)[::-1].copy(),
                 45 + n)

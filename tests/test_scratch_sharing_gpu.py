@@ -17,7 +17,7 @@ from tests.util import down, up, up_f16
 pytestmark = pytest.mark.gpu
 
 
-def test_every_decode_kind_through_one_scratch(gpu):
+def test_every_decode_kind_through_one_scratch(gpu, monkeypatch):
     from ttsxabe_amd.gpu import DecodeScratch, KvCacheQ8
 
     calls = []
@@ -44,13 +44,25 @@ def test_every_decode_kind_through_one_scratch(gpu):
         return lambda s: down(gpu.attn_decode_q8_batch(q, cache, tkd, sld, int(max(tk)), heads, hd ** -0.5, False, s))
 
     calls.append(("f16 32/8/128 tk 4096 (one XCD per head)", f16_case(32, 8, 128, 4096, 4096, 900)))
-    calls.append(("q8 batch of 5 (stream-K)", q8_case(128, 32, 8, 5, 2048, [2000, 31, 1500, 700, 2048], 901)))
+    # The two grids of a batch count their arrivals in the same counters, each
+    # in its own encoding.
+    batch = q8_case(128, 32, 8, 5, 2048, [2000, 31, 1500, 700, 2048], 901)
+
+    def stream_k(s):
+        with monkeypatch.context() as m:
+            m.setenv("LLMTIE_DECODE_STATIC", "0")
+            return batch(s)
+
+    calls.append(("q8 batch of 5 (stream-K)", stream_k))
+    calls.append(("q8 batch of 5 (planned grid)", batch))
     calls.append(("f16 4/2/128 tk 16500 (two-phase merge)", f16_case(4, 2, 128, 16500, 16512, 902)))
     calls.append(("f32 8/8/64 tk 5000", f32_case(8, 8, 64, 5000, 5056, 903)))
     calls.append(("q8 batch of 70 (planned grid)", q8_case(128, 8, 2, 70, 320, list(range(5, 285, 4)), 904)))
+    calls.append(("q8 batch of 5 (stream-K), again", stream_k))
     calls.append(("f16 40/40/128 tk 1500", f16_case(40, 40, 128, 1500, 1536, 905)))
 
     fresh = [fn(DecodeScratch()) for _, fn in calls]
+    assert not np.array_equal(fresh[1], fresh[2]), "two grids"
     shared = DecodeScratch()
     for rep in range(3):
         for (name, fn), want in zip(calls, fresh):
