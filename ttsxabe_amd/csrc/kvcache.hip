@@ -179,7 +179,7 @@ __global__ __launch_bounds__(KB) void append_vt_kernel(const float* src, T* dst,
     for (int r = 0; r < AT_P * AT_D / 4 / KB; ++r) {
         const int e = (int)threadIdx.x + r * KB;
         const int q = e % (AT_D / 4), pl = e / (AT_D / 4);
-        const int ti = p0 + pl - past;
+        const int ti = pl + (p0 - past);  // p0 + pl may pass an int
         if (ti < 0 || ti >= n) continue;
         const float4 x = *reinterpret_cast<const float4*>(src + (size_t)ti * d + d0 + 4 * q);
         tile[4 * q][pl] = x.x;
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(KB) void append_vt_kernel(const float* src, T* dst,
     for (int r = 0; r < AT_P * AT_D / 4 / KB; ++r) {
         const int e = (int)threadIdx.x + r * KB;
         const int pl = e % (AT_P / 4) * 4, dl = e / (AT_P / 4);
-        const int ti = p0 + pl - past;
+        const int ti = pl + (p0 - past);
         T* at = dst + (size_t)(d0 + dl) * cap + p0 + pl;
         quad y;
 #pragma unroll
@@ -220,7 +220,6 @@ __global__ __launch_bounds__(KB) void append_vt_kernel(const float* src, T* dst,
 // block maxima on DPP, not LDS shuffles) 2.77 -> 2.56.
 //
 // The pair of element e of a row of heads, rotated at position p.
-template <int HD>
 __device__ __forceinline__ float2 rotated_pair(const float* row, int hh, int j, int hd, float theta, const float* div,
                                                int p) {
     const int half = hd >> 1;
@@ -243,7 +242,7 @@ __global__ __launch_bounds__(KB) void rope_cache_f16_kernel(float* q, const floa
         const bool is_q = i < nq;
         const int e = is_q ? i : i - nq;
         const int j = e % half, hh = e / half;
-        const float2 y = rotated_pair<HD>(is_q ? q : k, hh, j, hd, theta, div, pos);
+        const float2 y = rotated_pair(is_q ? q : k, hh, j, hd, theta, div, pos);
         if (is_q) {
             float* d = q + (size_t)hh * hd + j;
             d[0] = y.x;
@@ -473,7 +472,7 @@ __global__ __launch_bounds__(KB) void rope_cache_q8_kernel(float* q, const float
         const int i = blockIdx.x * KB + threadIdx.x;
         if (i >= nq) return;
         const int j = i % half, hh = i / half;
-        const float2 y = rotated_pair<HD>(q, hh, j, hd, theta, div, pos);
+        const float2 y = rotated_pair(q, hh, j, hd, theta, div, pos);
         float* d = q + (size_t)hh * hd + j;
         d[0] = y.x;
         d[half] = y.y;
@@ -486,7 +485,7 @@ __global__ __launch_bounds__(KB) void rope_cache_q8_kernel(float* q, const float
     const int hh = e / hd, jj = e % hd;
     float x = 0.0f;
     if (live && is_k) {
-        const float2 y = rotated_pair<HD>(k, hh, jj % half, hd, theta, div, pos);
+        const float2 y = rotated_pair(k, hh, jj % half, hd, theta, div, pos);
         x = jj < half ? y.x : y.y;
     } else if (live) {
         x = v[e];
@@ -600,7 +599,7 @@ __global__ __launch_bounds__(KB) void rope_cache_t16_kernel(float* q, const floa
         const bool is_q = i < nq;
         const int e = is_q ? i : i - nq;
         const int j = e % half, hh = e / half;
-        const float2 y = rotated_pair<HD>(is_q ? q : k, hh, j, hd, theta, div, pos);
+        const float2 y = rotated_pair(is_q ? q : k, hh, j, hd, theta, div, pos);
         if (is_q) {
             float* d = q + (size_t)hh * hd + j;
             d[0] = y.x;

@@ -505,29 +505,29 @@ __device__ __forceinline__ void softmax_tile(floatx4 (&sc)[2][2][NQT], int u, in
     l += ps;
 }
 
-// Stores columns col0 .. col0 + WD - 1 of the context rows row0 .. row0 + 15
-// (query tile u of the wave; rows >= tq skipped) in line order: the wave's O /
-// l goes through its private LDS region R (16 x WD floats, a row's 16-byte chunk c at position
-// c ^ (row & SW), so both the fragment-order writes and the row-order reads
+// Stores the context rows row0 .. row0 + 15 of head h (query tile u of the
+// wave; rows >= tq skipped) in line order: the wave's O / l goes through its
+// private LDS region R (16 x HD floats, a row's 16-byte chunk c at position
+// c ^ (row & 15), so both the fragment-order writes and the row-order reads
 // hit 16 different bank groups per 16 lanes), and each store instruction
 // then writes whole lines (LPR lanes a row) instead of 16 rows' half lines
 // (C3 at 512 rows 13.43 -> 13.31 us, at 128 rows 6.28 -> 6.16 us).
-template <int WD, int NQT>
-__device__ __forceinline__ void store_ctx16(float* R, const floatx4 (&o)[WD / 16][NQT], int u, float inv, int lane,
-                                            const PrefillArgs& a, int row0, int col0) {
-    constexpr int NT = WD / 16, LPR = WD / 4, RPI = 64 / LPR, SW = LPR < 16 ? LPR - 1 : 15;
+template <int HD, int NQT>
+__device__ __forceinline__ void store_ctx16(float* R, const floatx4 (&o)[HD / 16][NQT], int u, float inv, int lane,
+                                            const PrefillArgs& a, int row0, int h) {
+    constexpr int NT = HD / 16, LPR = HD / 4, RPI = 64 / LPR;
     const int col = lane & 15, grp = lane >> 4;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         const float4 y = make_float4(o[t][u][0] * inv, o[t][u][1] * inv, o[t][u][2] * inv, o[t][u][3] * inv);
-        *reinterpret_cast<float4*>(R + col * WD + 4 * ((4 * t + grp) ^ (col & SW))) = y;
+        *reinterpret_cast<float4*>(R + col * HD + 4 * ((4 * t + grp) ^ col)) = y;
     }
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         const int row = i * RPI + lane / LPR, c = lane % LPR;
-        const float4 x = *reinterpret_cast<const float4*>(R + row * WD + 4 * (c ^ (row & SW)));
+        const float4 x = *reinterpret_cast<const float4*>(R + row * HD + 4 * (c ^ (row & 15)));
         if (row0 + row < a.tq) {
-            const size_t off = (size_t)(row0 + row) * a.os + (size_t)col0 + 4 * c;
+            const size_t off = (size_t)(row0 + row) * a.os + (size_t)h * HD + 4 * c;
             if (a.out_f16) {
                 half4 y;
                 y[0] = to_h(x.x); y[1] = to_h(x.y); y[2] = to_h(x.z); y[3] = to_h(x.w);
@@ -1065,7 +1065,7 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(Prefi
                 // row's (m, l) behind the runs' contexts.
                 PrefillArgs w = a;
                 w.out = a.ws + (size_t)sp * a.tq * a.os;
-                store_ctx16<HD, NQT>(R, o, u, 1.0f, lane, w, p0 + 16 * u, h * HD);
+                store_ctx16<HD, NQT>(R, o, u, 1.0f, lane, w, p0 + 16 * u, h);
                 const int r = p0 + 16 * u + col;
                 if (grp == 0 && r < a.tq) {
                     float2* ml = reinterpret_cast<float2*>(a.ws + (size_t)a.splits * a.tq * a.os);
@@ -1073,7 +1073,7 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, 8 / W) void flash_fwd_kernel(Prefi
                 }
                 continue;
             }
-            store_ctx16<HD, NQT>(R, o, u, lt > 0.0f ? 1.0f / lt : 0.0f, lane, a, p0 + 16 * u, h * HD);
+            store_ctx16<HD, NQT>(R, o, u, lt > 0.0f ? 1.0f / lt : 0.0f, lane, a, p0 + 16 * u, h);
         }
         return;
     }
