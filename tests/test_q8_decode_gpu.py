@@ -218,3 +218,27 @@ def test_batches_run_on_the_grid_that_is_faster(gpu, hd, heads, kv, nseq, high, 
     sk = run()
     assert np.array_equal(got, sk) == stream_k
     assert full_scale_err(sk, got) < 2e-3  # each within 1e-3 of the exact value
+
+
+# Batches of few and of many blocks a wave on the planned grid, which the
+# default rule takes for them.
+@pytest.mark.parametrize("hd,heads,kv,lengths", [
+    (128, 32, 8, [1590, 801, 1233]), (128, 32, 8, [2202, 1500]), (64, 32, 8, [2681, 300, 900, 2000, 1411, 77]),
+    (128, 16, 4, [3000, 2999, 64, 1025])])
+def test_the_planned_grid_is_no_further_off_than_stream_k(gpu, hd, heads, kv, lengths, monkeypatch):
+    from ttsxabe_amd.gpu import DecodeScratch, KvCacheQ8
+    n, cap, each = len(lengths), max(lengths), heads * hd
+    parts = random_q8_cache(n, kv, hd, cap, 71)
+    cache = KvCacheQ8(n, kv, hd, cap)
+    load(cache, *parts)
+    q = oracle.normal(n * each, 78)
+    slot = np.arange(n, dtype=np.int32)
+    run = lambda: down(gpu.attn_decode_q8_batch(up(q), cache, up(np.array(lengths, np.int32), torch.int32),
+                                                up(slot, torch.int32), cap, heads, hd ** -0.5, False, DecodeScratch()))
+    planned = run()
+    monkeypatch.setenv("LLMTIE_DECODE_STATIC", "0")
+    sk = run()
+    exact = np.concatenate([oracle.decode_f64(q[i * each:(i + 1) * each], *dequant_seq(*parts, i, kv, hd, cap), heads,
+                                              kv, hd, tk, cap, hd ** -0.5, False) for i, tk in enumerate(lengths)])
+    assert not np.array_equal(planned, sk)
+    assert np.linalg.norm(planned - exact) <= np.linalg.norm(sk - exact)

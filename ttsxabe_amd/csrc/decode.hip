@@ -265,8 +265,9 @@ __device__ __forceinline__ half_t h_at(const uint4& u, int e) {
 }
 
 // One 32-key block folded into the wave's running softmax state. MASK: keys
-// >= tk are dropped (only the partial block needs it).
-template <int HD, int KIND, bool MASK>
+// >= tk are dropped (only the partial block needs it). ONCE (Q8_0): P' below
+// is rounded once.
+template <int HD, int KIND, bool MASK, bool ONCE = false>
 __device__ __forceinline__ void fold_block(const Frag<HD, KIND>& f, const half8 (&qh)[HD / 32],
                                            const half8 (&ql)[HD / 32],
                                            int p0, int tk, int grp,
@@ -345,6 +346,13 @@ __device__ __forceinline__ void fold_block(const Frag<HD, KIND>& f, const half8 
         // per dim block, formed with packed f16 multiplies: Q8_0 values carry
         // 8 bits, so the 11 of an f16 P' keep the product well inside the
         // quantisation's own error.
+        // ONCE: formed in f32 and rounded once, not P first. A batch of up to 64
+        // sequences has waves of more blocks on this grid than under stream-K,
+        // so fewer of its heaviest keys are a wave's maximum, whose P is exact:
+        // with P rounded first its error was 1.02 of stream-K's over 36 drawn
+        // batches, at most 1.055; rounded once it is 0.74, at most 0.77. At 8 kv
+        // heads of 128: 8 sequences of 256-4096, 17.0 us before and 17.1 so; 3
+        // of 800-1590, 9.16 / 9.31; 32 of 100-1000, 12.2 / 12.5.
         typedef _Float16 h2 __attribute__((ext_vector_type(2)));
         h2 ph[4];
 #pragma unroll
@@ -365,7 +373,12 @@ __device__ __forceinline__ void fold_block(const Frag<HD, KIND>& f, const half8 
                     if (kb + 2 * i >= tk) d[0] = (half_t)0.0f;
                     if (kb + 2 * i + 1 >= tk) d[1] = (half_t)0.0f;
                 }
-                const h2 x = ph[i] * d;
+                h2 x = ph[i] * d;
+                if constexpr (ONCE) {
+                    // p of a masked key is 0 and its d zeroed above
+                    x = h2{to_h(__builtin_fmaf(p[2 * i], (float)d[0], 0.0f)),
+                           to_h(__builtin_fmaf(p[2 * i + 1], (float)d[1], 0.0f))};
+                }
                 pv[2 * i] = x[0];
                 pv[2 * i + 1] = x[1];
             }
@@ -417,7 +430,7 @@ __device__ __forceinline__ void fold_block(const Frag<HD, KIND>& f, const half8 
 }
 
 // One tiled Q8_0 block folded into the wave's running softmax state: the
-// arithmetic of fold_block<HD, KV_TQ8>, bit for bit, in an order that keeps
+// arithmetic of fold_block<HD, KV_TQ8> (ONCE off), bit for bit, in an order that keeps
 // the matrix unit and the VALU busy together (one wave per SIMD issues a
 // VALU instruction only every ~6-7 clocks, so the stream-K kernel's blocks
 // cost their VALU count). Every K fragment is dequantised first; the sixteen
@@ -954,8 +967,9 @@ __device__ __forceinline__ bool one_xcd(unsigned long long c) {
 // W waves a workgroup: 4, or 8 for a context of one split and 5 to 16 blocks
 // (a.waves). There a wave's chain of folds is what the launch waits for, and
 // nothing is handed to another workgroup, so twice the waves halve it (the
-// times stand at the plan's rule, one_split_blocks).
-template <int HD, int KIND, int VA, bool G1, int W = DW>
+// times stand at the plan's rule, one_split_blocks). ONCE: Q8_0 batches of up to
+// 64 sequences (fold_block).
+template <int HD, int KIND, int VA, bool G1, int W = DW, bool ONCE = false>
 __global__ __launch_bounds__(W * LLMTIE_WAVE, KIND == KV_F32 ? 1 : 2) void attn_decode_kernel(DecodeArgs a) {
     constexpr int DW = W, DT = W * LLMTIE_WAVE;  // this launch's (the merge's are four waves')
     constexpr int NS = HD / 32;
@@ -1100,7 +1114,7 @@ __global__ __launch_bounds__(W * LLMTIE_WAVE, KIND == KV_F32 ? 1 : 2) void attn_
         else if constexpr (G1)
             fold_block_g1<HD, KIND, MASK>(f, qv, p, tk, col, grp, m_run, l_run, o1, prow[wave]);
         else
-            fold_block<HD, KIND, MASK>(f, qh, ql, p, tk, grp, a.score_l2, m_run, l_run, o);
+            fold_block<HD, KIND, MASK, ONCE>(f, qh, ql, p, tk, grp, a.score_l2, m_run, l_run, o);
     };
 
     // Two blocks in flight: while block i is folded, block i + 1 is on its
@@ -2122,6 +2136,8 @@ DECODE_INST2(64, KV_F16, 16) DECODE_INST2(128, KV_F16, 16) DECODE_INST2(64, KV_F
 DECODE_INST2(64, KV_F32, 16) DECODE_INST2(128, KV_F32, 16) DECODE_INST2(64, KV_F32, 8)
 DECODE_INST2(128, KV_F32, 8) DECODE_INST2(64, KV_T16, 16) DECODE_INST2(128, KV_T16, 16)
 DECODE_INST(64, KV_TQ8, 16, false) DECODE_INST(128, KV_TQ8, 16, false)
+template __global__ void attn_decode_kernel<64, KV_TQ8, 16, false, DW, true>(DecodeArgs);
+template __global__ void attn_decode_kernel<128, KV_TQ8, 16, false, DW, true>(DecodeArgs);
 
 template __global__ void attn_decode_sk_kernel<64>(DecodeArgs);
 template __global__ void attn_decode_sk_kernel<128>(DecodeArgs);
@@ -2169,6 +2185,11 @@ static hipError_t launch_attn(int hd, int kind, const DecodeArgs& a, int kv_head
     }
 #undef L82
 #undef L8
+    if (kind == KV_TQ8 && nseq <= 64) {
+        if (hd == 128) hipLaunchKernelGGL((attn_decode_kernel<128, KV_TQ8, 16, false, DW, true>), grid, block, 0, st, b);
+        else hipLaunchKernelGGL((attn_decode_kernel<64, KV_TQ8, 16, false, DW, true>), grid, block, 0, st, b);
+        return hipGetLastError();
+    }
 #define L(HD, KIND, VA, G1)                                                                    \
     if (hd == HD && kind == KIND && va == VA && g1 == G1) {                                    \
         hipLaunchKernelGGL((attn_decode_kernel<HD, KIND, VA, G1>), grid, block, 0, st, b);      \
