@@ -422,3 +422,38 @@ def test_rows_quantised_in_whole_chunks_are_the_rows_quantised_alone(gpu, n, pas
     for t in range(n):
         gpu.kv_q8_append(dk, t * kv * hd, dv, t * kv * hd, alone, slot, 1, past + t)
     assert torch.equal(whole.data, alone.data)
+
+
+@pytest.mark.parametrize("kind", ["t16_k", "t16_v", "q8"])
+def test_two_rows_of_the_most_heads_a_launch_takes(gpu, kind):
+    """Two rows over two blocks of 2^23 heads of 64: as whole chunks their
+    workgroups would reach a launch's 2^32 threads, element by element they are
+    a quarter of that."""
+    from ttsxabe_amd.gpu import KvCacheQ8, TiledCache16
+    kv, hd, cap, n, past = 2**23, 64, 64, 2, 31
+    src = torch.empty(n * kv * hd, device="cuda").uniform_(-1.0, 1.0)
+    if kind == "q8":
+        cache = KvCacheQ8.__new__(KvCacheQ8)
+        cache.slots, cache.kv_heads, cache.head_dim, cache.cap = 1, kv, hd, cap
+        per = KvCacheQ8(1, 1, hd, cap).data.numel()
+        cache.data = torch.empty(kv * per, dtype=torch.int8, device="cuda")
+        one = lambda: KvCacheQ8(1, 1, hd, cap)
+        append = lambda s, c: gpu.kv_q8_append(s, 0, s, 0, c, 0, n, past)
+    else:
+        cache = TiledCache16(kv, hd, cap, zero=False)
+        per = cache.data.numel() // kv
+        one = lambda: TiledCache16(1, hd, cap)
+        append = lambda s, c: gpu.t16_append(s, 0, c, n, past, kind == "t16_v")
+    at = (0, 1, kv // 2 - 1, kv // 2, kv - 2, kv - 1)
+    for h in at:
+        cache.data[h * per:(h + 1) * per].copy_(one().data)
+    append(src, cache)
+    bad = []
+    for h in at:
+        want = one()
+        append(src.view(n, kv, hd)[:, h].contiguous().view(-1), want)
+        if not torch.equal(cache.data[h * per:(h + 1) * per], want.data):
+            bad.append(h)
+    del cache, src
+    torch.cuda.empty_cache()
+    assert not bad

@@ -632,6 +632,11 @@ __global__ __launch_bounds__(KB) void ref_to_t16_kernel(const uint16_t* k, const
 }
 
 static inline unsigned nblk(long n) { return (unsigned)((n + KB - 1) / KB); }
+// Workgroups of an append in whole chunks: a wave a unit, then the edges'
+// elements. Past CHUNK_WGS a launch would reach 2^32 threads (two to seven rows
+// over two blocks of half a billion dims), where the flat form still has room.
+static inline long chunk_wgs(long units, long edges) { return (units + KB / 64 - 1) / (KB / 64) + (edges + KB - 1) / KB; }
+constexpr long CHUNK_WGS = (1L << 32) / KB - 1;
 static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 hipError_t launch_rope(float* x, long off, const float* div, int t, int heads, int hd, float theta, int first,
@@ -737,8 +742,9 @@ hipError_t launch_append_q8(const float* k, long k_off, const float* v, long v_o
     const long units = (long)((past + n - 1) / 32 - b0 + 1) * kv * (hd / 16);
     // As launch_append_t16, from half as many elements (there are two areas):
     // 60 rows of 8 x 128, 3.59 us in chunks and 3.44 flat; 173 rows, 3.64 and 3.87.
-    if (tot >= 1L << 17 && aligned16(k + k_off) && aligned16(cache) && hd % 64 == 0 && units <= 0x7fffffffL - KB) {
-        const dim3 g((unsigned)((units + KB / 64 - 1) / (KB / 64)) + nblk((long)Edges(past, n).count() * kv * hd));
+    const long wgs = chunk_wgs(units, (long)Edges(past, n).count() * kv * hd);
+    if (tot >= 1L << 17 && aligned16(k + k_off) && aligned16(cache) && hd % 64 == 0 && wgs <= CHUNK_WGS) {
+        const dim3 g((unsigned)wgs);
         hipLaunchKernelGGL(append_q8_chunks_kernel, g, dim3(KB), 0, st, k + k_off, v + v_off, cache, slot, n, kv, hd, tiled_nblk(cap), past, (int)units, b0);
         return hipGetLastError();
     }
@@ -771,9 +777,9 @@ hipError_t launch_append_t16(const float* src, long src_off, uint16_t* cache, in
     // Whole chunks once the flat form would take about 1024 workgroups (V) or
     // from two rows on (K, whose chunks are one key's): 173 rows of 8 x 128, V
     // 2.66 us in chunks and 2.57 flat; 300 rows, 3.17 and 3.31; K even at 29.
-    if ((value ? tot >= 1L << 18 : n > 1) && aligned16(src + src_off) && aligned16(cache) && hd % 64 == 0 && units <= 0x7fffffffL - KB) {
-        const dim3 g((unsigned)((units + KB / 64 - 1) / (KB / 64)) +
-                     (value ? nblk((long)Edges(past, n).count() * kv * hd) : 0u));
+    const long wgs = chunk_wgs(units, value ? (long)Edges(past, n).count() * kv * hd : 0);
+    if ((value ? tot >= 1L << 18 : n > 1) && aligned16(src + src_off) && aligned16(cache) && hd % 64 == 0 && wgs <= CHUNK_WGS) {
+        const dim3 g((unsigned)wgs);
         if (value) hipLaunchKernelGGL((append_t16_chunks_kernel<true>), g, dim3(KB), 0, st, src + src_off, cache, n, kv, hd, tiled_nblk(cap), past, (int)units, b0);
         else hipLaunchKernelGGL((append_t16_chunks_kernel<false>), g, dim3(KB), 0, st, src + src_off, cache, n, kv, hd, tiled_nblk(cap), past, (int)units, b0);
         return hipGetLastError();
