@@ -200,7 +200,9 @@ def test_stream_k_and_the_planned_grid_are_the_same_attention(gpu, hd, heads, kv
 # that it is faster on: stream-K's bits are its own.
 @pytest.mark.parametrize("hd,heads,kv,nseq,high,stream_k", [
     (128, 32, 8, 17, 1646, True), (128, 16, 8, 25, 1050, True), (128, 40, 40, 4, 1281, True),
-    (128, 40, 40, 3, 2276, True), (128, 32, 8, 14, 1681, False), (128, 16, 8, 19, 1060, False),
+    (128, 40, 40, 3, 2276, True), (128, 32, 8, 18, 1135, True), (128, 32, 8, 17, 1027, True),
+    (128, 16, 8, 19, 1060, True), (64, 32, 8, 60, 1096, True), (128, 32, 8, 14, 1681, False),
+    (128, 16, 8, 19, 1000, False), (64, 32, 8, 47, 1263, False),
     (64, 32, 8, 17, 1129, False), (128, 16, 8, 54, 471, False)])
 def test_batches_run_on_the_grid_that_is_faster(gpu, hd, heads, kv, nseq, high, stream_k, monkeypatch):
     from ttsxabe_amd.gpu import DecodeScratch, KvCacheQ8

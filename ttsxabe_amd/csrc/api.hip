@@ -363,11 +363,11 @@ void plan_decode(size_t tk_max, size_t units, size_t group, int& nit, int& split
 // Stream-K balances ragged lengths, but each wave holds a head's pieces, so a
 // batch of few blocks pays for merging hundreds of them: the host only knows
 // the lengths' bound, so the line is drawn at the bytes that it allows. Host
-// plan / stream-K, us, at 8 kv heads of 128: 1 sequence of 4000, 9.2 / 42.8; 4 of
-// 500-2000, 10.3 / 22.7; 8 of 256-4096 (bound 71 MB), 16.4 / 25.6; 8 of
-// 6000-8000 (139 MB), 28 / 36; 32 of 100-1000 (70 MB), 14.2 / 18.3; 12 of
-// 20-8000 (209 MB), 37-44 / 33; 16 of 500-4000 (139 MB), 25-30 / 28; 32 of
-// 256-8192 (570 MB), 71 / 58.8. More than 64 sequences always take the plan.
+// plan / stream-K, us, at 8 kv heads of 128: 1 sequence of 4000, 8.6 / 42.6; 4 of
+// 500-2000, 9.8 / 22.1; 8 of 256-4096 (bound 71 MB), 15.2 / 23.0; 8 of
+// 6000-8000 (139 MB), 25.9 / 34.1; 32 of 100-1000 (70 MB), 12.4 / 16.7; 12 of
+// 20-8000 (209 MB), 45 / 35; 16 of 500-4000 (139 MB), 28 / 23; 32 of 256-8192
+// (570 MB), 68 / 54.6. More than 64 sequences always take the plan.
 bool plan_q8_batch(size_t nseq, size_t kv_heads, size_t hd, size_t max_tk, int& nit, int& splits) {
     const char* e = getenv("LLMTIE_DECODE_STATIC");
     if (nseq > 64 || (e && atoi(e))) return false;
@@ -376,20 +376,21 @@ bool plan_q8_batch(size_t nseq, size_t kv_heads, size_t hd, size_t max_tk, int& 
     const double mb = (double)units * (double)max_tk * (double)(2 * hd + hd / 8) * 1e-6;
     if (mb > (units <= 64 ? 150.0 : 75.0)) return true;
     // Beyond one round of workgroups, even spans of up to 1024 keys (eight blocks
-    // a wave): 12 sequences of 100-1000, 10.8 us against 14.0 in three splits
-    // each; 20, 12.6 / 15.5; 32, 14.2 / 20.9.
+    // a wave): 12 sequences of 100-1000, 11.0 us against 14.0 in three splits
+    // each; 20, 12.2 / 14.4; 32, 12.4 / 17.2.
     if (units > 64 && units * (size_t)splits > 256 && nit < 8 && !getenv("LLMTIE_DECODE_NIT") &&
         !getenv("LLMTIE_DECODE_WGS")) {
         const size_t spans = (max_tk + 1023) / 1024;
         nit = (int)(((max_tk + 31) / 32 + 4 * spans - 1) / (4 * spans));
         splits = (int)((max_tk + 128 * (size_t)nit - 1) / (128 * (size_t)nit));
     }
-    // Several such rounds of split heads at head_dim 128 lose to stream-K from
-    // 45 MB on: 17 sequences of up to 1646 over 8 kv heads, 23.8 / 20.5 us; 25 of
-    // 1050, 21.4 / 18.9; 19 of 1174 (48 MB), 19.2 / 17.8; 4 of 1281 over 40, 20.4 /
-    // 18.9; but 14 of 1681 over 8 (one round), 17.8 / 21.0; 19 of 1088 (45 MB),
-    // 15.6 / 16.8.
-    return hd == 128 && splits > 1 && units * (size_t)splits > 256 && mb > 45.0;
+    // Split heads past one workgroup a compute unit (three at head_dim 64, which
+    // fit side by side) lose to stream-K. Over 8 kv heads of 128: 17 sequences of
+    // up to 1646, 23.8 / 20.5 us; 18 of 283-1135, 17.8 / 16.2; 17 of 924-1027, 18.2
+    // / 17.1; but 16 of 529-1059 (256 workgroups), 14.0 / 16.6. Of 64: 60 of
+    // 274-1096, 21.7 / 19.7; 53 of 263-1054 (848 workgroups), 19.0 / 17.9; but 47 of
+    // 1136-1263 (752), 16.7 / 22.0.
+    return splits > 1 && units * (size_t)splits > (hd == 64 ? 768 : 256);
 }
 
 // Whether the split partials are merged by a second launch rather than by
