@@ -137,10 +137,10 @@ int llmtie_flash_attn_f16(void* stream, const float* q, size_t q_len, const uint
  * needs (0: the shape is not split, and no workspace is needed; never more than
  * 64 * 16 * (head_dim + 2) a compute unit, 136 MB at head_dim 128). The workspace
  * is written and read on `stream` by this call alone and may be reused or
- * freed in stream order after it; concurrent calls need one each. `ws` NULL is
- * the plain call. A workspace shorter than needed is refused as
- * LLMTIE_SLICE_OVERRUN, one that is not 16-byte aligned as
- * LLMTIE_INVALID_ARGUMENT. */
+ * freed in stream order after it; concurrent calls need one each. Split, the
+ * context is the plain call's to rounding. `ws` NULL is the plain call. A
+ * workspace shorter than needed is refused as LLMTIE_SLICE_OVERRUN, one that is
+ * not 16-byte aligned as LLMTIE_INVALID_ARGUMENT. */
 size_t llmtie_flash_attn_workspace(size_t tq, size_t past, size_t heads, size_t kv_heads, size_t head_dim);
 int llmtie_flash_attn_f16_ws(void* stream, const float* q, size_t q_len, const uint16_t* k, size_t k_len,
                              const uint16_t* v, size_t v_len, float* out, size_t out_len, size_t tq, size_t past,
@@ -213,7 +213,8 @@ int llmtie_attn_decode(void* stream, const float* q, size_t q_len, const float* 
  * arrays; max_tk bounds every tk_dev[s] (the kernel clamps to it, never
  * reading past it) and must be <= cap. A sequence whose slot is out of range
  * or whose length is 0 gets a NaN row. cache_len is in bytes
- * (llmtie_q8_cache_bytes). */
+ * (llmtie_q8_cache_bytes). Up to 64 sequences max_tk also decides how the keys
+ * are divided over the chip: results under two bounds agree to rounding. */
 int llmtie_attn_decode_q8_batch(void* stream, const float* q, size_t q_len, const int8_t* cache, size_t cache_len,
                                 size_t slots, const int32_t* tk_dev, const int32_t* slot_dev, size_t nseq,
                                 size_t max_tk, size_t heads, size_t kv_heads, size_t head_dim, size_t cap,

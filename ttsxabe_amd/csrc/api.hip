@@ -869,7 +869,7 @@ int llmtie_attn_decode_q8_batch(void* stream, const float* q, size_t q_len, cons
     // Up to 64 sequences the hand-off is coherent on either grid: no head of
     // such a batch can be lost. XCD-local / coherent on the planned grid: 8
     // sequences of 256-4096 at 32/8/128, a step of 8 layers 290 / 297 us; 20 of
-    // 386-1042 at 32/8/64, four layers 47.2 / 42.9; nine other batches within 1 %.
+    // 386-1042 at 32/8/64, four layers 47.2 / 42.9; nine other batches within 2 %.
     a.xcd = sk || nseq <= 64 ? 0 : xcd_local(splits, kv_heads * nseq, a.two_phase);
     a.xcd_fake = g_fake_xcc.load() ? 1 : 0;
     a.lost = scratch->lost;
