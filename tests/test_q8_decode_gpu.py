@@ -16,8 +16,8 @@ from tests.util import down, full_scale_err, up
 pytestmark = pytest.mark.gpu
 
 
-# A batch of up to 64 sequences runs on the host-planned grid or stream-K by the
-# bytes its length bound allows: the default rule, and stream-K forced.
+# A batch of up to 64 sequences runs on the host-planned grid or stream-K by its
+# shape and length bound: the default rule, and stream-K forced.
 both_grids = pytest.mark.parametrize("static", [None, "0"])
 
 
